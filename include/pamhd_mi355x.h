@@ -375,7 +375,8 @@ pamhd_set_launch) is called a handle uses the variants it picks for the
 256^3 HLLD step: XCD-aware flux block order, HLLD's per-cell part carried
 along 16-cell marches in all three directions, the z-marching update with 8
 planes per 128 x 2 tile (grids of fewer than 16 planes: per-face flux
-kernels and the per-cell update).  (No counterpart in the reference.)
+kernels and the per-cell update); grids of up to 2^20 cells (HLLD: 2^22) run
+the flat step instead (pamhd_set_launch).  (No counterpart in the reference.)
 */
 int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen,
 	void* stream);
@@ -387,7 +388,10 @@ int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen,
    along marches of 16 cells for the y- and z-faces (bit 5: 4 cells), bit 6
    = as bit 4 and the x-faces marched along y too, each lane's part moved to
    the next lane (bits 3-6 for HLLD, bits 4-6 also for HLL and Rusanov
-   on grids without a background field; bit 1 is then ignored);
+   on grids without a background field; bit 1 is then ignored), bit 7 = the
+   flat step: one launch for all faces and one for all cells whatever the
+   grid's size (the default of grids too small for marches to fill the GPU;
+   the other bits and arguments are then ignored);
    update_remap bits 0 and 1 the same
    orders for the update pass (bit 0 only for the z-marching update) and,
    for the z-marching update, bits 2-4 its tile (0: 64 x 4, 1: 128 x 2,

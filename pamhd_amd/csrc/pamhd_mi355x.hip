@@ -68,6 +68,18 @@ struct StepStatus {
 	int err;
 	long long err_face;
 	unsigned long long flux_calcs;   /* faces solved (substepping path) */
+	/* flat step: face index * 16 + error code of the first failed face in
+	   index order, ERR_KEY_NONE without one */
+	unsigned long long err_key;
+};
+constexpr unsigned long long ERR_KEY_NONE = ~0ull;
+
+/* the step length and, for the flat step, the reduced speeds of the last
+   flux pass that the next lagged step length comes from */
+struct DtRec {
+	double dt;
+	double smax[3];
+	unsigned zero[3];
 };
 
 constexpr int BX = 64, BY = 4;      /* flux pass and cell kernels */
@@ -1075,27 +1087,19 @@ __global__ __launch_bounds__(TX * TY) void update_column_kernel(GridDev g,
 }
 
 /*
-Per-cell update variant (one thread per cell, no marching): the same sums in
-the same order as update_column_kernel, recomputing the positive-side faces'
-dB instead of carrying them between planes; also the kernel of the z-slab
-pipeline.
+The update of one cell: the same sums in the same order as
+update_column_kernel, recomputing the positive-side faces' dB instead of
+carrying them between planes.
 */
 template <class PT>
-__global__ __launch_bounds__(BX * BY) void update_cell_kernel(GridDev g,
-	const double* __restrict__ s, double* __restrict__ out,
-	const PT* __restrict__ P, int refits, unsigned gx, unsigned gy, int remap, int k0,
+__device__ __forceinline__ void update_cell(const GridDev& g, const double* __restrict__ s,
+	double* __restrict__ out, const PT* __restrict__ P, int refits, int i, int j, int kk,
 	double* __restrict__ pe)
 {
-	const unsigned lb = (remap & 1) ? logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
-	unsigned bx, by, k;
-	tile_of_block(lb, gx, gy, gridDim.x, remap, k0, bx, by, k);
-	const int i = bx * BX + threadIdx.x;
-	const int j = by * BY + threadIdx.y;
-	if (i >= g.nx || j >= g.ny) return;
 	const long long n = g.n;
 	const int im = wrap_dec(i, g.nx), ip = wrap_inc(i, g.nx);
 	const int jm = wrap_dec(j, g.ny), jp = wrap_inc(j, g.ny);
-	const int kk = (int)k, km = wrap_dec(kk, g.nz), kp = wrap_inc(kk, g.nz), kpp = wrap_inc(kp, g.nz);
+	const int km = wrap_dec(kk, g.nz), kp = wrap_inc(kk, g.nz);
 	const Nb L{g.nx, g.ny};
 	const EdgeTerms<PT> E{P, n, g.dx, g.dy, g.dz};
 	const double axy = g.dx * g.dy, axz = g.dx * g.dz, ayz = g.dy * g.dz;
@@ -1110,7 +1114,6 @@ __global__ __launch_bounds__(BX * BY) void update_cell_kernel(GridDev g,
 	out[5 * n + c] = bx_new;
 	out[6 * n + c] = by_new;
 	out[7 * n + c] = bz_new;
-	(void)kpp;
 
 	const long long cp[3] = {cxp, cyp, czp};
 	double rho = s[c];
@@ -1159,6 +1162,236 @@ __global__ __launch_bounds__(BX * BY) void update_cell_kernel(GridDev g,
 			return (double)P[((long long)d * 8 + q) * n + c];
 		});
 	}
+}
+
+/* per-cell update (one thread per cell, no marching); also the kernel of
+   the z-slab pipeline */
+template <class PT>
+__global__ __launch_bounds__(BX * BY) void update_cell_kernel(GridDev g,
+	const double* __restrict__ s, double* __restrict__ out,
+	const PT* __restrict__ P, int refits, unsigned gx, unsigned gy, int remap, int k0,
+	double* __restrict__ pe)
+{
+	const unsigned lb = (remap & 1) ? logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
+	unsigned bx, by, k;
+	tile_of_block(lb, gx, gy, gridDim.x, remap, k0, bx, by, k);
+	const int i = bx * BX + threadIdx.x;
+	const int j = by * BY + threadIdx.y;
+	if (i >= g.nx || j >= g.ny) return;
+	update_cell<PT>(g, s, out, P, refits, i, j, (int)k, pe);
+}
+
+/*
+Flat step: two launches, for grids too small to fill the GPU with marches
+(flat_step).  A thread takes one face (flat_flux_kernel, the three
+directions of a run of cells in neighbouring blocks of one launch) or one
+cell (flat_update_kernel) of the flat index, so no lane idles at the end of
+a short row.  The first launch computes the lagged step length itself from
+the speeds that the previous step's second launch reduced, and the second
+launch's last block reduces this step's speeds for the next one, so there
+is no step-length launch in between and the host reads the step's result
+from memory that block wrote.
+
+What bounds a small step is the chain of launches and of each thread's
+dependent FP64 operations: a step of the 20 x 20 HLL grid ran five launches
+and two copies, 41 us, of which 31 us in kernels that follow one another.
+*/
+
+/* flat index / d for indexes below 2^28: (c * m) >> sh, with
+   sh = 28 + ceil(log2 d) and m = floor(2^sh / d) + 1 < 2^29 + 1 (exact by
+   the usual argument: the error c (m d - 2^sh) / (d 2^sh) < 1 / d) */
+struct FlatDiv {
+	unsigned m, sh;
+	__device__ __forceinline__ unsigned operator()(unsigned c) const
+	{
+		return (unsigned)(((unsigned long long)c * m) >> sh);
+	}
+};
+
+struct FlatGrid {
+	FlatDiv nx, ny;
+	__device__ __forceinline__ void cell(const GridDev& g, int c, int& i, int& j, int& k) const
+	{
+		const unsigned t = nx((unsigned)c);
+		i = c - (int)t * g.nx;
+		k = (int)ny(t);
+		j = (int)t - k * g.ny;
+	}
+};
+
+__device__ __forceinline__ void record_error_ordered(StepStatus* st, int code, long long face)
+{
+	atomicMin(&st->err_key, (unsigned long long)face * 16 + (unsigned)code);
+}
+
+/* load_face_state_d with the direction known at run time (the same in the
+   whole block): rotated components by uniform offsets */
+__device__ __forceinline__ void load_face_state(const double* __restrict__ s, const GridDev& g,
+	int d, int i, int j, int k, double U[8])
+{
+	const size_t n = (size_t)g.n;
+	const int c = i + g.nx * (j + g.ny * k);
+	const int d1 = d == 2 ? 0 : d + 1, d2 = d1 == 2 ? 0 : d1 + 1;
+	const int up[3] = {wrap_inc(i, g.nx) + g.nx * (j + g.ny * k),
+		i + g.nx * (wrap_inc(j, g.ny) + g.ny * k), i + g.nx * (j + g.ny * wrap_inc(k, g.nz))};
+	const int u0 = d == 0 ? up[0] : d == 1 ? up[1] : up[2];
+	const int u1 = d == 0 ? up[1] : d == 1 ? up[2] : up[0];
+	const int u2 = d == 0 ? up[2] : d == 1 ? up[0] : up[1];
+	const double *b0 = s + (5 + d) * n, *b1 = s + (5 + d1) * n, *b2 = s + (5 + d2) * n;
+	U[RHO] = s[c];
+	U[M0] = (s + (1 + d) * n)[c];
+	U[M1] = (s + (1 + d1) * n)[c];
+	U[M2] = (s + (1 + d2) * n)[c];
+	U[NRJ] = (s + 4 * n)[c];
+	U[B0] = 0.5 * (b0[c] + b0[u0]);
+	U[B1] = 0.5 * (b1[c] + b1[u1]);
+	U[B2] = 0.5 * (b2[c] + b2[u2]);
+}
+
+/* the step length of dt_kernel from the reduced speeds */
+__device__ __forceinline__ double lagged_dt(const DtRec* __restrict__ rec, const GridDev& g,
+	double cfl, double max_dt, int fixed)
+{
+	if (fixed) return max_dt;
+	const double len[3] = {g.dx, g.dy, g.dz};
+	double cfl_dt = DBL_MAX;
+	for (int d = 0; d < 3; d++) {
+		if (rec->zero[d] > 0) {
+			cfl_dt = 0;
+			break;
+		}
+		cfl_dt = smin(cfl_dt, cfl * len[d] / rec->smax[d]);
+	}
+	return max_dt <= cfl_dt ? max_dt : cfl_dt;
+}
+
+constexpr int FLAT = BX * BY;   /* threads per block of the flat kernels */
+
+template <int SOLVER, class T>
+__global__ __launch_bounds__(FLAT) void flat_flux_kernel(GridDev g, FlatGrid fg,
+	const double* __restrict__ s, const double* __restrict__ bg, double* __restrict__ P,
+	DtRec* __restrict__ rec, double cfl, double max_dt, int fixed, StepStatus* st)
+{
+	const int d = (int)(blockIdx.x % 3);
+	const int c = (int)(blockIdx.x / 3) * FLAT + threadIdx.x;
+	double sp = 0;
+	unsigned zero = 0;
+	if (c < (int)g.n) {
+		int i, j, k;
+		fg.cell(g, c, i, j, k);
+		const int li = d == 0 ? wrap_dec(i, g.nx) : i, lj = d == 1 ? wrap_dec(j, g.ny) : j,
+			lk = d == 2 ? wrap_dec(k, g.nz) : k;
+		double L[8], R[8];
+		load_face_state(s, g, d, li, lj, lk, L);
+		load_face_state(s, g, d, i, j, k, R);
+		const double step = lagged_dt(rec, g, cfl, max_dt, fixed);
+		if (c == 0 && d == 0) rec->dt = step;
+		const int d1 = d == 2 ? 0 : d + 1, d2 = d1 == 2 ? 0 : d1 + 1;
+		T b[3] = {0, 0, 0};
+		if (bg) {
+			/* Bg_B(L)(+d): the face is the positive d-face of L */
+			const int cl = li + g.nx * (lj + g.ny * lk);
+			const double* bgd = bg + (size_t)(3 * d) * g.n;
+			b[0] = (T)bgd[(size_t)d * g.n + cl];
+			b[1] = (T)bgd[(size_t)d1 * g.n + cl];
+			b[2] = (T)bgd[(size_t)d2 * g.n + cl];
+		}
+		/* dt * F in the precisions of flux_pass_kernel */
+		using FT = std::conditional_t<SOLVER == HLLD_ATHENA, double, T>;
+		FT F[8], sT = 0;
+		int e;
+		if constexpr (SOLVER == HLLD_ATHENA && std::is_same_v<T, float>) {
+			e = riemann_d<SOLVER, T>(L, R, b, g.ph, F, sT);
+		} else {
+			e = riemann<SOLVER, T>(L, R, b, g.ph, F, sT);
+		}
+		const FT dt = (FT)step;
+		if (e) {
+			record_error_ordered(st, e, (long long)d * g.n + c);
+#pragma unroll
+			for (int q = 0; q < 8; q++) F[q] = 0;
+			sT = 0;
+		} else {
+#pragma unroll
+			for (int q = 0; q < 8; q++) F[q] = dt * F[q];
+		}
+		const size_t n = (size_t)g.n;
+		double* Pd = P + (size_t)d * 8 * n;
+		Pd[c] = (double)F[RHO];
+		(Pd + (1 + d) * n)[c] = (double)F[M0];
+		(Pd + (1 + d1) * n)[c] = (double)F[M1];
+		(Pd + (1 + d2) * n)[c] = (double)F[M2];
+		(Pd + 4 * n)[c] = (double)F[NRJ];
+		(Pd + (5 + d) * n)[c] = (double)F[B0];
+		(Pd + (5 + d1) * n)[c] = (double)F[B1];
+		(Pd + (5 + d2) * n)[c] = (double)F[B2];
+		sp = (double)sT;
+		zero = sp <= 0 ? 1u : 0u;
+	}
+	reduce_speed(st, d, sp, zero);
+}
+
+/* lane s reduces slot s of every dimension and clears the other status
+   entry for the next flux pass; the speeds of the pass that wrote `cur` go
+   to rec (the same ordered bit patterns as dt_kernel) */
+__device__ __forceinline__ void reduce_lag(StepStatus* __restrict__ cur,
+	StepStatus* __restrict__ other, DtRec* __restrict__ rec, int lane)
+{
+	for (int d = 0; d < 3; d++) {
+		unsigned long long m = cur->smax_bits[d][lane];
+		for (int off = NSLOT / 2; off > 0; off >>= 1) {
+			const unsigned long long o = __shfl_xor(m, off, NSLOT);
+			m = m < o ? o : m;
+		}
+		other->smax_bits[d][lane] = 0;
+		if (lane == 0) {
+			rec->smax[d] = __longlong_as_double((long long)m);
+			rec->zero[d] = cur->zero[d];
+			other->zero[d] = 0;
+		}
+	}
+	if (lane == 0) {
+		other->err = 0;
+		other->err_face = -1;
+		other->err_key = ERR_KEY_NONE;
+	}
+}
+
+/* before the first flat step after another one */
+__global__ __launch_bounds__(NSLOT) void lag_kernel(StepStatus* cur, StepStatus* other, DtRec* rec)
+{
+	reduce_lag(cur, other, rec, threadIdx.x);
+}
+
+/* cells / FLAT blocks update the cells, the last block ends the pass; host
+   (pinned, may be null) receives the step length and the error */
+__global__ __launch_bounds__(FLAT) void flat_update_kernel(GridDev g, FlatGrid fg,
+	const double* __restrict__ s, double* __restrict__ out, const double* __restrict__ P, int refits,
+	double* __restrict__ pe, StepStatus* cur, StepStatus* other, DtRec* rec, double* host_dt,
+	StepStatus* host)
+{
+	if (blockIdx.x + 1 == gridDim.x) {
+		if (threadIdx.x >= NSLOT) return;
+		reduce_lag(cur, other, rec, threadIdx.x);
+		if (threadIdx.x == 0) {
+			const unsigned long long key = cur->err_key;
+			const int err = key == ERR_KEY_NONE ? 0 : (int)(key & 15);
+			const long long face = err ? (long long)(key >> 4) : -1;
+			cur->err = err;
+			cur->err_face = face;
+			if (host) {
+				*host_dt = rec->dt;
+				host->err = err;
+				host->err_face = face;
+			}
+		}
+		return;
+	}
+	const int c = (int)blockIdx.x * FLAT + threadIdx.x;
+	if (c >= (int)g.n) return;
+	int i, j, k;
+	fg.cell(g, c, i, j, k);
+	update_cell<double>(g, s, out, P, refits, i, j, k, pe);
 }
 
 /*
@@ -1994,6 +2227,7 @@ __global__ __launch_bounds__(NSLOT) void dt_kernel(const StepStatus* __restrict_
 	for (int d = 0; d < 3; d++) next->zero[d] = 0;
 	next->err = 0;
 	next->err_face = -1;
+	next->err_key = ERR_KEY_NONE;
 }
 
 /* energy refit of apply_boundaries for a periodic grid (update_vol_B with
@@ -3223,10 +3457,10 @@ struct pamhd_handle {
 	double* state[2] = {nullptr, nullptr};
 	double* flux = nullptr;
 	double* bg = nullptr;
-	double* dt = nullptr;
+	double* dt = nullptr;         /* a DtRec; its first member is the step length */
 	double* scratch = nullptr;
 	size_t scratch_len = 0;
-	StepStatus* status = nullptr; /* 2 entries */
+	StepStatus* status = nullptr; /* 2 entries, and one that pamhd_autotune may overwrite */
 	double* host_dt = nullptr;    /* pinned */
 	StepStatus* host_status = nullptr;
 	/* launch choices, set by pamhd_autotune (defaults: per-cell update) */
@@ -3253,7 +3487,11 @@ struct pamhd_handle {
 		int fused = -1;
 		int fused_kc = 16;     /* planes per chunk of the fused pass (<= FKC_MAX) */
 		int acc_km = 32;       /* cells per march of the accumulating step */
+		/* the flat step (two launches): 1 always, 0 never, -1 where the grid
+		   is small (flat_step) and no launch variant was asked for */
+		int flat = -1;
 	} tune;
+	bool lag_ok = false;   /* dt holds the last flux pass's reduced speeds and the other status is cleared */
 	double* emf = nullptr;     /* 6 x n field components of the fused step, allocated on first use */
 	/* second stream and events of the slab pipeline, created on first use */
 	hipStream_t aux = nullptr;
@@ -3594,6 +3832,64 @@ int launch_accumulate(pamhd_handle* h, hipStream_t st, StepStatus* next, int ref
 	}
 	HIP_TRY(h, hipGetLastError());
 	return launch_ct_refit(h, st, s, out, refits);
+}
+
+FlatDiv flat_div(unsigned d)
+{
+	unsigned lg = 0;
+	while ((1u << lg) < d) lg++;
+	const unsigned sh = 28 + lg;
+	return FlatDiv{(unsigned)(((1ull << sh) / d) + 1), sh};
+}
+
+/*
+Whether the step runs flat (see flat_flux_kernel) unless the caller chose.
+The marches and column updates keep less in the flux array and compute
+HLLD's per-cell part once, but put 32 cells in a thread: below ~10^6 cells
+they leave SIMDs without a wave.  us per step, marches -> flat:
+  HLLD  20x20 157 -> 13, 64^3 397 -> 66, 96^3 416 -> 210, 128^3 555 -> 498,
+        160^3 1068 -> 938, 192^3 1515 -> 1562
+  HLL   20x20 26 -> 12, 64^3 139 -> 54, 96^3 238 -> 170, 128^3 376 -> 418
+  Roe   20x20 33 -> 15, 64^3 101 -> 82, 96^3 328 -> 267, 128^3 605 -> 621
+so HLLD crosses over between 160^3 and 192^3, the others between 96^3 and
+128^3.  Kernel timing keeps the launches it accounts for.
+*/
+bool flat_step(const pamhd_handle* h, int solver)
+{
+	if (h->timing) return false;
+	if (h->tune.flat >= 0) return h->tune.flat == 1;
+	return h->g.n <= (solver == HLLD_ATHENA ? 1ll << 22 : 1ll << 20);
+}
+
+template <class T>
+int launch_flat(pamhd_handle* h, int solver, hipStream_t st, double max_dt, double cfl, int refits,
+	int fixed_dt, bool report, StepStatus* prev, StepStatus* next, StepStatus* clear)
+{
+	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+	(void)hipStreamIsCapturing(st, &cap);
+	const bool captured = cap != hipStreamCaptureStatusNone;
+	DtRec* rec = reinterpret_cast<DtRec*>(h->dt);
+	/* a captured step may run after any other one: it reduces the speeds
+	   itself, and so does the step after the capture */
+	if (!h->lag_ok || captured) lag_kernel<<<1, NSLOT, 0, st>>>(prev, next, rec);
+	const FlatGrid fg{flat_div((unsigned)h->g.nx), flat_div((unsigned)h->g.ny)};
+	const unsigned nb = (unsigned)((h->g.n + FLAT - 1) / FLAT);
+	const double* s = h->state[h->cur];
+#define FLUX(SV) flat_flux_kernel<SV, T><<<3 * nb, FLAT, 0, st>>>(h->g, fg, s, h->bg, h->flux, rec, cfl, \
+	max_dt, fixed_dt, next)
+	switch (solver) {
+	case RUSANOV: FLUX(RUSANOV); break;
+	case HLL_ATHENA: FLUX(HLL_ATHENA); break;
+	case HLLD_ATHENA: FLUX(HLLD_ATHENA); break;
+	default: FLUX(ROE_ATHENA); break;
+	}
+#undef FLUX
+	flat_update_kernel<<<nb + 1, FLAT, 0, st>>>(h->g, fg, s, h->state[1 - h->cur], h->flux, refits,
+		std::is_same_v<T, double> ? h->pe_out : nullptr, next, clear, rec, h->host_dt,
+		report ? h->host_status : nullptr);
+	h->lag_ok = !captured;
+	HIP_TRY(h, hipGetLastError());
+	return PAMHD_OK;
 }
 
 /*
@@ -4119,23 +4415,35 @@ int do_step(pamhd_handle* h, int solver, double max_dt, double cfl, int refits,
 	}
 	StepStatus* prev = h->status + h->last;
 	StepStatus* next = h->status + (1 - h->last);
-	{
-		TimedLaunch t(h, st, K_DT);
-		dt_kernel<<<1, NSLOT, 0, st>>>(prev, next, h->dt, cfl, max_dt, h->g.dx, h->g.dy, h->g.dz, fixed_dt);
+	const bool flat = flat_step(h, solver);
+	if (flat) {
+		const bool report = dt_taken != nullptr;
+		const int e = h->precision == PAMHD_MIXED
+			? launch_flat<float>(h, solver, st, max_dt, cfl, refits, fixed_dt, report, prev, next, prev)
+			: launch_flat<double>(h, solver, st, max_dt, cfl, refits, fixed_dt, report, prev, next, prev);
+		if (e) return e;
+	} else {
+		h->lag_ok = false;
+		{
+			TimedLaunch t(h, st, K_DT);
+			dt_kernel<<<1, NSLOT, 0, st>>>(prev, next, h->dt, cfl, max_dt, h->g.dx, h->g.dy, h->g.dz, fixed_dt);
+		}
+		HIP_TRY(h, hipGetLastError());
+		const int e = h->precision == PAMHD_MIXED
+			? launch_step_body<float, double>(h, solver, st, next, refits)
+			: launch_step_body<double, double>(h, solver, st, next, refits);
+		if (e) return e;
+		HIP_TRY(h, hipGetLastError());
 	}
-	HIP_TRY(h, hipGetLastError());
-	const int e = h->precision == PAMHD_MIXED
-		? launch_step_body<float, double>(h, solver, st, next, refits)
-		: launch_step_body<double, double>(h, solver, st, next, refits);
-	if (e) return e;
-	HIP_TRY(h, hipGetLastError());
 	h->flux_step = (h->precision == PAMHD_FP64 && !fused_step(h, solver)) ? 1 : 0;
 	h->cur = 1 - h->cur;
 	h->last = 1 - h->last;
 	h->flux_calcs = 3ull * (unsigned long long)h->g.n;
 	if (dt_taken) {
-		HIP_TRY(h, hipMemcpyAsync(h->host_dt, h->dt, sizeof(double), hipMemcpyDeviceToHost, st));
-		HIP_TRY(h, hipMemcpyAsync(h->host_status, next, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
+		if (!flat) {
+			HIP_TRY(h, hipMemcpyAsync(h->host_dt, h->dt, sizeof(double), hipMemcpyDeviceToHost, st));
+			HIP_TRY(h, hipMemcpyAsync(h->host_status, next, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
+		}
 		HIP_TRY(h, hipStreamSynchronize(st));
 		*dt_taken = *h->host_dt;
 		return report_status(h, *h->host_status);
@@ -4193,8 +4501,8 @@ int pamhd_create(const pamhd_grid_desc* grid, const pamhd_physics* physics, int 
 	if ((e = hipMalloc(&h->state[0], sizeof(double) * 8 * n)) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "state", e);
 	if ((e = hipMalloc(&h->state[1], sizeof(double) * 8 * n)) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "state", e);
 	if ((e = hipMalloc(&h->flux, sizeof(double) * 24 * n)) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "flux", e);
-	if ((e = hipMalloc(&h->dt, sizeof(double))) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "dt", e);
-	if ((e = hipMalloc(&h->status, 2 * sizeof(StepStatus))) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "status", e);
+	if ((e = hipMalloc(&h->dt, sizeof(DtRec))) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "dt", e);
+	if ((e = hipMalloc(&h->status, 3 * sizeof(StepStatus))) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "status", e);
 	if ((e = hipHostMalloc(&h->host_dt, sizeof(double))) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "pinned", e);
 	if ((e = hipHostMalloc(&h->host_status, sizeof(StepStatus))) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "pinned", e);
 	/* before the first flux pass every face's Max_v is -1
@@ -4207,6 +4515,7 @@ int pamhd_create(const pamhd_grid_desc* grid, const pamhd_physics* physics, int 
 		}
 		s.err = 0;
 		s.err_face = -1;
+		s.err_key = ERR_KEY_NONE;
 	}
 	if ((e = hipMemcpy(h->status, init, sizeof(init), hipMemcpyHostToDevice)) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "status", e);
 	if ((e = hipMemset(h->state[0], 0, sizeof(double) * 8 * n)) != hipSuccess) return cleanup(PAMHD_E_DEVICE, "state", e);
@@ -4920,6 +5229,7 @@ int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen, void* 
 	hipStream_t st = (hipStream_t)stream_;
 	const bool timing = h->timing;
 	h->timing = false;
+	h->lag_ok = false;
 	StepStatus* prev = h->status + h->last;
 	StepStatus* next = h->status + (1 - h->last);
 	hipEvent_t a, b;
@@ -5074,12 +5384,30 @@ int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen, void* 
 			h->tune = best_t;
 		}
 	}
+	/* the flat step against the step chosen so far */
+	{
+		const float ms = time_it([&]() {
+			dt_kernel<<<1, NSLOT, 0, st>>>(prev, next, h->dt, 0.0, 0.0, h->g.dx, h->g.dy, h->g.dz, 0);
+			if (h->precision == PAMHD_MIXED) launch_step_body<float, double>(h, solver, st, next, 3);
+			else launch_step_body<double, double>(h, solver, st, next, 3);
+		});
+		h->lag_ok = false;
+		const float flat_ms = time_it([&]() {
+			if (h->precision == PAMHD_MIXED)
+				launch_flat<float>(h, solver, st, 0.0, 0.0, 3, 0, false, prev, next, h->status + 2);
+			else
+				launch_flat<double>(h, solver, st, 0.0, 0.0, 3, 0, false, prev, next, h->status + 2);
+		});
+		h->lag_ok = false;
+		h->tune.flat = flat_ms < ms ? 1 : 0;
+		report += "; marches=" + std::to_string(ms) + "ms flat=" + std::to_string(flat_ms) + "ms";
+	}
 	(void)hipEventDestroy(a);
 	(void)hipEventDestroy(b);
 	HIP_TRY(h, hipGetLastError());
 	HIP_TRY(h, hipStreamSynchronize(st));
 	h->timing = timing;
-	report += "; chosen fused=" + std::to_string(h->tune.fused) +
+	report += "; chosen " + std::string(h->tune.flat ? "flat " : "") + "fused=" + std::to_string(h->tune.fused) +
 		(h->tune.fused == 1 ? "/kc" + std::to_string(h->tune.fused_kc) :
 		 h->tune.fused == 2 ? "/km" + std::to_string(h->tune.acc_km) : std::string()) +
 		" flux_remap=" + std::to_string(h->tune.flux_remap) +
@@ -5106,6 +5434,7 @@ int pamhd_set_launch(pamhd_handle* h, int flux_remap, int update_kz, int update_
 	h->tune.update_kz = update_kz;
 	h->tune.update_remap = update_kz ? (update_remap & 1) : (update_remap & 3);
 	h->tune.update_tile = update_kz ? (update_remap >> 2) % 5 : 0;
+	h->tune.flat = (flux_remap & 128) ? 1 : 0;
 	return PAMHD_OK;
 }
 
@@ -5118,6 +5447,7 @@ int pamhd_set_fused_step(pamhd_handle* h, int fused, int planes_per_chunk)
 	if (planes_per_chunk < 0 || planes_per_chunk > most)
 		return fail(h, PAMHD_E_ARG, "planes per chunk must be in 0.." + std::to_string(most));
 	h->tune.fused = fused;
+	h->tune.flat = fused < 0 ? -1 : 0;
 	if (planes_per_chunk > 0) {
 		if (fused == 2) h->tune.acc_km = planes_per_chunk;
 		else h->tune.fused_kc = planes_per_chunk;
@@ -5131,6 +5461,7 @@ int pamhd_set_slabs(pamhd_handle* h, int slabs)
 	if (!h) return fail(nullptr, PAMHD_E_ARG, "null handle");
 	if (slabs < 1) return fail(h, PAMHD_E_ARG, "slabs must be >= 1");
 	h->tune.slabs = slabs;
+	if (slabs > 1) h->tune.flat = 0;
 	return PAMHD_OK;
 }
 
