@@ -375,8 +375,8 @@ pamhd_set_launch) is called a handle uses the variants it picks for the
 256^3 HLLD step: XCD-aware flux block order, HLLD's per-cell part carried
 along 16-cell marches in all three directions, the z-marching update with 8
 planes per 128 x 2 tile (grids of fewer than 16 planes: per-face flux
-kernels and the per-cell update); grids of up to 2^20 cells (HLLD: 2^22) run
-the flat step instead (pamhd_set_launch).  (No counterpart in the reference.)
+kernels and the per-cell update); grids of up to 2^20 cells run the
+flat step instead (pamhd_set_launch).  (No counterpart in the reference.)
 */
 int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen,
 	void* stream);
@@ -409,7 +409,8 @@ int pamhd_set_launch(pamhd_handle* h, int flux_remap, int update_kz, int update_
    and finish with a pass that updates the face field and refits the
    energy.  -1 (the default) picks 2; pamhd_autotune times them all.
    planes_per_chunk (0 = keep) is the z-extent of mode 1's blocks (1..32)
-   or the cells per march of mode 2 (1..32). */
+   or the cells per march of mode 2 (1..32; until it is given they follow
+   the grid's size). */
 int pamhd_set_fused_step(pamhd_handle* h, int fused, int planes_per_chunk);
 
 /* Pipelines the flux pass and the per-cell update over `slabs` z-slabs on

@@ -1872,11 +1872,11 @@ Accumulating step (HLLD): the three per-direction marches of the two-pass
 path, each finishing its direction's part of update_mhd_state's conserved
 update (source/mhd/solve.hpp:1503-1614) instead of storing face fluxes:
 
-  acc_x_kernel      x-faces, a wave per 64-cell x tile walking km rows along
-                    y (the left part of lane l is lane l - 1's, the face of
-                    lane l + 1 comes one lane down; the tile's left-edge parts
-                    and right-edge face fluxes are computed for all km rows
-                    before the march, one row per lane); writes
+  acc_x_kernel      x-faces, a wave per 64 cells of a plane walking km planes
+                    along z (the left part of lane l is lane l - 1's, the
+                    face of lane l + 1 comes one lane down; the rows'
+                    left-edge parts and right-edge face fluxes are computed
+                    for all km planes before the march); writes
                     out = U + x terms (8 values: rho, m, E, cell-centred B)
   acc_march_kernel  y- (D = 1) and z-faces (D = 2), a thread walking km cells
                     of a line along D with the part of the cell just walked
@@ -1971,81 +1971,114 @@ template <int D> __device__ __forceinline__ void store_emf(double* __restrict__ 
 	}
 }
 
-constexpr int ACC_KMAX = 32;   /* cells per march of the accumulating x pass, at most */
+constexpr int ACC_KMAX = 32;   /* cells per march that a caller may ask for, at most */
+constexpr int ACC_EDGE = 64;   /* row edges x planes that a wave of the x pass keeps in LDS */
 
+/* the rows that 64 consecutive cells of a plane touch, at most: each has a
+   left edge cell and a right edge face of its own */
+__host__ __device__ __forceinline__ int acc_segments(int nx)
+{
+	return nx % BX == 0 ? 1 : (BX - 2) / nx + 2;
+}
+
+/*
+x-faces.  A wave takes 64 consecutive cells of the plane's flat index
+i + nx j and marches km planes along z, so rows that are no multiple of 64
+cells leave no lane idle (nx = 200: 22 % of the lanes of 64-cell row tiles).
+Where a row starts inside the wave the left part is not the lane below's,
+and where one ends the right face is not the lane above's: those, and the
+wave's own first and last, are computed for all km planes before the march,
+one edge and plane per lane (acc_segments(nx) * km <= ACC_EDGE).  Mixed
+200 x 180 x 152 step, row tiles -> flat index (both marches): x 365 -> 304,
+y 391 -> 267, z 301 -> 242 us.
+*/
 template <class T, int MINB>
-__global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, StateArrays S,
+__global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv div_nx, StateArrays S,
 	double* __restrict__ out, double* __restrict__ emf, const double* __restrict__ dtp,
 	StepStatus* st, unsigned gx, int km, int remap)
 {
-	static_assert(BX == 64, "a wave is one x tile");
+	static_assert(BX == 64, "a wave is 64 cells");
 	using P = typename APartOf<T>::type;
 	const unsigned lb = (remap & 1) ? logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
-	const unsigned gt = (unsigned)((g.nz + BY - 1) / BY);
-	const unsigned bx = lb % gx, r = lb / gx;
-	const int kk = (int)(r % gt) * BY + threadIdx.y;
-	const int chunk = (int)(r / gt);
+	const unsigned bx = lb % gx;
+	const int chunk = (int)(lb / gx);
 	const int lane = threadIdx.x;
 	const int tid = lane + BX * threadIdx.y;
-	const int i0 = (int)bx * BX;
-	const int i = (i0 + lane) % g.nx;         /* lanes past the grid wrap */
-	const bool own_x = i0 + lane < g.nx;
+	const int plane = g.nx * g.ny;
+	/* the wave's first cell of the plane, its row and column */
+	const int l0 = __builtin_amdgcn_readfirstlane((int)(bx * BY + threadIdx.y) * BX);
+	const int j0 = (int)div_nx((unsigned)l0), i0 = l0 - j0 * g.nx;
+	const bool own = l0 + lane < plane;
+	const int l = min(l0 + lane, plane - 1);   /* lanes past the plane repeat its last cell */
+	const int j = (int)div_nx((unsigned)l), i = l - j * g.nx;
+	const int seg = j - j0;
+	const bool row_start = i == 0, row_end = i + 1 == g.nx;
 	const int a0 = chunk * km;
-	const int a1 = min(a0 + km, g.ny);
+	const int a1 = min(a0 + km, g.nz);
 	const size_t n = g.n;
 	double sp = 0;
 	unsigned zero = 0;
-	/* per wave: the tile's left-edge parts and right-edge face fluxes of
-	   the march's rows, and each lane's face flux (read by the lane below) */
-	__shared__ P edge_l[BY][ACC_KMAX];
-	__shared__ Flux8<double> edge_r[BY][ACC_KMAX];
+	/* per wave: the left-edge parts and right-edge face fluxes of its rows
+	   and planes, and each lane's face flux (read by the lane below) */
+	__shared__ P edge_l[BY][ACC_EDGE];
+	__shared__ Flux8<double> edge_r[BY][ACC_EDGE];
 	__shared__ double lo_s[8][BX * BY];
-	/* kk, a0 and a1 are the same in every lane of the wave */
-	if (kk < g.nz && a0 < a1) {
+	/* l0, a0 and a1 are the same in every lane of the wave */
+	if (l0 < plane && a0 < a1) {
 		const double dt = *dtp;
 		const double il = 1 / g.dx;
-		if (lane < a1 - a0) {
-			const int row = a0 + lane;
+		const int planes = a1 - a0;
+		const int segs = min((i0 + BX - 1) / g.nx + 1, g.ny - j0);
+		if (lane < segs * planes) {
+			const int sg = lane / planes, a = a0 + lane % planes;
+			const int row = j0 + sg;
+			const int first = sg == 0 ? i0 : 0;
+			const int last = min(i0 + BX - 1 - sg * g.nx, g.nx - 1);
 			double U[8];
-			load_face_state_d<0>(S, g, wrap_dec(i0, g.nx), row, kk, U);
+			load_face_state_d<0>(S, g, wrap_dec(first, g.nx), row, a, U);
 			apart_make<T>(U, g.ph, edge_l[threadIdx.y][lane]);
-			if (i0 + BX <= g.nx) {
-				P pa, pb;
-				load_face_state_d<0>(S, g, i0 + BX - 1, row, kk, U);
-				apart_make<T>(U, g.ph, pa);
-				load_face_state_d<0>(S, g, (i0 + BX) % g.nx, row, kk, U);
-				apart_make<T>(U, g.ph, pb);
-				double s_unused;
-				apart_face<T, 0>(pa, pb, g.ph, dt, edge_r[threadIdx.y][lane].f, s_unused);
-			}
+			P pa, pb;
+			load_face_state_d<0>(S, g, last, row, a, U);
+			apart_make<T>(U, g.ph, pa);
+			load_face_state_d<0>(S, g, wrap_inc(last, g.nx), row, a, U);
+			apart_make<T>(U, g.ph, pb);
+			double s_unused;
+			apart_face<T, 0>(pa, pb, g.ph, dt, edge_r[threadIdx.y][lane].f, s_unused);
 		}
 		__builtin_amdgcn_wave_barrier();
 		for (int a = a0; a < a1; a++) {
 			double s_face;
 			int e;
+			const int at = a - a0, mine = min(seg, segs - 1) * planes + at;
 			if constexpr (std::is_same_v<T, double>) {
 				/* FP64: the face of the lane above comes down with a DPP
-				   wavefront shift (lane 63 takes the tile's right-edge
+				   wavefront shift (lane 63 takes the wave's right-edge
 				   face); every lane of the wave is active here */
 				double lo[8], hi[8];
 				{
 					double U[8];
-					load_face_state_d<0>(S, g, i, a, kk, U);
+					load_face_state_d<0>(S, g, i, j, a, U);
 					P R;
 					apart_make<T>(U, g.ph, R);
-					const P L = apart_up(R, edge_l[threadIdx.y][a - a0]);
+					P L = apart_up(R, edge_l[threadIdx.y][at]);
+					if (row_start) L = edge_l[threadIdx.y][mine];
 					e = apart_face<T, 0>(L, R, g.ph, dt, lo, s_face);
 				}
 #pragma unroll
-				for (int q = 0; q < 8; q++) hi[q] = lane_down_dpp(lo[q], edge_r[threadIdx.y][a - a0].f[q]);
-				if (own_x) {
-					const int c = i + g.nx * (a + g.ny * kk);
+				for (int q = 0; q < 8; q++)
+					hi[q] = lane_down_dpp(lo[q], edge_r[threadIdx.y][(segs - 1) * planes + at].f[q]);
+				if (row_end) {
+#pragma unroll
+					for (int q = 0; q < 8; q++) hi[q] = edge_r[threadIdx.y][mine].f[q];
+				}
+				if (own) {
+					const int c = l + plane * a;
 					double U[8];
 					if (e) record_error(st, e, (long long)c);
 					sp = smax(sp, s_face);
 					zero += s_face <= 0 ? 1u : 0u;
 					store_emf<0>(emf, n, c, lo);
-					load_face_state_d<0>(S, g, i, a, kk, U);
+					load_face_state_d<0>(S, g, i, j, a, U);
 					add_terms<double>(U, lo, hi, g.dx, il);
 #pragma unroll
 					for (int q = 0; q < 8; q++) out[q * n + c] = U[q];
@@ -2054,10 +2087,11 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, StateAr
 			}
 			{
 				double U[8];
-				load_face_state_d<0>(S, g, i, a, kk, U);
+				load_face_state_d<0>(S, g, i, j, a, U);
 				P R;
 				apart_make<T>(U, g.ph, R);
-				const P L = apart_up(R, edge_l[threadIdx.y][a - a0]);
+				P L = apart_up(R, edge_l[threadIdx.y][at]);
+				if (row_start) L = edge_l[threadIdx.y][mine];
 				double lo[8];
 				e = apart_face<T, 0>(L, R, g.ph, dt, lo, s_face);
 #pragma unroll
@@ -2069,21 +2103,21 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, StateAr
 			   held in registers across the face */
 			__asm__ volatile("" ::: "memory");
 			__builtin_amdgcn_wave_barrier();
-			if (own_x) {
-				const int c = i + g.nx * (a + g.ny * kk);
+			if (own) {
+				const int c = l + plane * a;
 				double lo[8], hi[8], U[8];
-				const bool last = lane == BX - 1;
+				const bool last = row_end || lane == BX - 1;
 				const int up = last ? tid : tid + 1;
 #pragma unroll
 				for (int q = 0; q < 8; q++) {
 					lo[q] = lo_s[q][tid];
-					hi[q] = last ? edge_r[threadIdx.y][a - a0].f[q] : lo_s[q][up];
+					hi[q] = last ? edge_r[threadIdx.y][mine].f[q] : lo_s[q][up];
 				}
 				if (e) record_error(st, e, (long long)c);
 				sp = smax(sp, s_face);
 				zero += s_face <= 0 ? 1u : 0u;
 				store_emf<0>(emf, n, c, lo);
-				load_face_state_d<0>(S, g, i, a, kk, U);
+				load_face_state_d<0>(S, g, i, j, a, U);
 				add_terms<double>(U, lo, hi, g.dx, il);
 #pragma unroll
 				for (int q = 0; q < 8; q++) out[q * n + c] = U[q];
@@ -2095,27 +2129,29 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, StateAr
 	reduce_speed(st, 0, sp, zero);
 }
 
+/* y- and z-faces: a thread marches km cells of a line along D; the lines
+   are taken by the flat index of the other two dimensions (x fastest), so
+   every lane has one whatever the row length */
 template <class T, int D, int MINB>
-__global__ __launch_bounds__(BX * BY, MINB) void acc_march_kernel(GridDev g, StateArrays S,
+__global__ __launch_bounds__(BX * BY, MINB) void acc_march_kernel(GridDev g, FlatDiv div_nx, StateArrays S,
 	double* __restrict__ out, double* __restrict__ emf, const double* __restrict__ dtp,
 	StepStatus* st, unsigned gx, int km, int remap, int refits)
 {
 	static_assert(D == 1 || D == 2, "march along y or z");
 	using P = typename APartOf<T>::type;
 	const unsigned lb = (remap & 1) ? logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
-	const int nt = D == 1 ? g.nz : g.ny;                 /* lines across */
-	const unsigned gt = (unsigned)((nt + BY - 1) / BY);
-	const unsigned bx = lb % gx, r = lb / gx;
-	const int t = (int)(r % gt) * BY + threadIdx.y;
-	const int chunk = (int)(r / gt);
-	const int i = bx * BX + threadIdx.x;
+	const int lines = g.nx * (D == 1 ? g.nz : g.ny);
+	const int line = (int)(lb % gx) * (BX * BY) + threadIdx.x + BX * threadIdx.y;
+	const int chunk = (int)(lb / gx);
+	const int t = (int)div_nx((unsigned)line);
+	const int i = line - t * g.nx;
 	const int nd = D == 1 ? g.ny : g.nz;
 	const int a0 = chunk * km;
 	const int a1 = min(a0 + km, nd);
 	const size_t n = g.n;
 	double sp = 0;
 	unsigned zero = 0;
-	if (i < g.nx && t < nt && a0 < a1) {
+	if (line < lines && a0 < a1) {
 		const int jj = D == 1 ? 0 : t;
 		const int kk = D == 1 ? t : 0;
 		const double dt = *dtp;
@@ -3486,7 +3522,7 @@ struct pamhd_handle {
 		   face-field update and refits), -1 = the default (2) */
 		int fused = -1;
 		int fused_kc = 16;     /* planes per chunk of the fused pass (<= FKC_MAX) */
-		int acc_km = 32;       /* cells per march of the accumulating step */
+		int acc_km = 0;        /* cells per march of the accumulating step, 0: march_cells */
 		/* the flat step (two launches): 1 always, 0 never, -1 where the grid
 		   is small (flat_step) and no launch variant was asked for */
 		int flat = -1;
@@ -3805,6 +3841,41 @@ int launch_fused(pamhd_handle* h, hipStream_t st, StepStatus* next, int refits)
 	return launch_ct_refit(h, st, s, out, refits);
 }
 
+FlatDiv flat_div(unsigned d)
+{
+	unsigned lg = 0;
+	while ((1u << lg) < d) lg++;
+	const unsigned sh = 28 + lg;
+	return FlatDiv{(unsigned)(((1ull << sh) / d) + 1), sh};
+}
+
+/*
+Cells per march of a pass over `blocks` blocks of lines with nd cells each,
+at most `most`, when `resident` blocks run on a CU at once: a march of km
+cells costs about km + 1.5 faces, and the blocks run in
+ceil(blocks * chunks / (256 * resident)) rounds, so a fixed km leaves CUs
+idle in the last round or altogether.  FP64 HLLD step, 32-cell marches ->
+this rule: 128^3 545 -> 412 us, 192^3 1493 -> 1387 us, 256^3 within 1 %
+(there VALU issue is the bound whatever the rounds).
+*/
+int march_cells(unsigned blocks, int nd, int resident, int most)
+{
+	const long long slots = 256ll * resident;
+	int best = 1;
+	double best_cost = 1e300;
+	for (int chunks = 1; chunks <= nd; chunks++) {
+		const int km = (nd + chunks - 1) / chunks;
+		if (km > most) continue;
+		const double cost = (double)((blocks * (long long)chunks + slots - 1) / slots) * (km + 1.5);
+		if (cost < best_cost) {
+			best_cost = cost;
+			best = km;
+		}
+		if (km == 1) break;
+	}
+	return best;
+}
+
 /* the accumulating step: x, y and z marches into state[1 - cur], then the
    face-field update and refits */
 template <class T>
@@ -3816,49 +3887,44 @@ int launch_accumulate(pamhd_handle* h, hipStream_t st, StepStatus* next, int ref
 	double* out = h->state[1 - h->cur];
 	StateArrays S;
 	for (int q = 0; q < 8; q++) S.q[q] = s + (size_t)q * n;
-	const int km = std::min(std::max(1, h->tune.acc_km), ACC_KMAX);
-	const unsigned gx = (h->g.nx + BX - 1) / BX;
-	const unsigned tz = (h->g.nz + BY - 1) / BY, ty = (h->g.ny + BY - 1) / BY;
-	const unsigned cy = (h->g.ny + km - 1) / km, cz = (h->g.nz + km - 1) / km;
 	const int r = h->tune.flux_remap;
 	const dim3 block(BX, BY, 1);
+	const FlatDiv dx = flat_div((unsigned)h->g.nx);
+	auto blocks = [](long long lines) { return (unsigned)((lines + BX * BY - 1) / (BX * BY)); };
+	const unsigned gxy = blocks((long long)h->g.nx * h->g.ny), gxz = blocks((long long)h->g.nx * h->g.nz);
+	/* x: 2 waves per SIMD resident, at most ACC_EDGE row edges per wave */
+	const int edges = std::max(1, ACC_EDGE / acc_segments(h->g.nx));
+	const int kx = h->tune.acc_km > 0 ? std::min(h->tune.acc_km, edges) : march_cells(gxy, h->g.nz, 2, std::min(edges, ACC_KMAX));
+	const int ky = h->tune.acc_km > 0 ? h->tune.acc_km : march_cells(gxz, h->g.ny, 3, ACC_KMAX);
+	const int kz = h->tune.acc_km > 0 ? h->tune.acc_km : march_cells(gxy, h->g.nz, 3, ACC_KMAX);
 	{
 		TimedLaunch t(h, st, K_FLUX);
-		acc_x_kernel<T, 1><<<gx * tz * cy, block, 0, st>>>(h->g, S, out, h->emf, h->dt, next, gx, km, r);
-		acc_march_kernel<T, 1, 3><<<gx * tz * cy, block, 0, st>>>(h->g, S, out, h->emf, h->dt, next,
-			gx, km, r, refits);
-		acc_march_kernel<T, 2, 3><<<gx * ty * cz, block, 0, st>>>(h->g, S, out, h->emf, h->dt, next,
-			gx, km, r, refits);
+		acc_x_kernel<T, 1><<<gxy * ((h->g.nz + kx - 1) / kx), block, 0, st>>>(h->g, dx, S, out, h->emf, h->dt,
+			next, gxy, kx, r);
+		acc_march_kernel<T, 1, 3><<<gxz * ((h->g.ny + ky - 1) / ky), block, 0, st>>>(h->g, dx, S, out, h->emf,
+			h->dt, next, gxz, ky, r, refits);
+		acc_march_kernel<T, 2, 3><<<gxy * ((h->g.nz + kz - 1) / kz), block, 0, st>>>(h->g, dx, S, out, h->emf,
+			h->dt, next, gxy, kz, r, refits);
 	}
 	HIP_TRY(h, hipGetLastError());
 	return launch_ct_refit(h, st, s, out, refits);
 }
 
-FlatDiv flat_div(unsigned d)
-{
-	unsigned lg = 0;
-	while ((1u << lg) < d) lg++;
-	const unsigned sh = 28 + lg;
-	return FlatDiv{(unsigned)(((1ull << sh) / d) + 1), sh};
-}
-
 /*
 Whether the step runs flat (see flat_flux_kernel) unless the caller chose.
 The marches and column updates keep less in the flux array and compute
-HLLD's per-cell part once, but put 32 cells in a thread: below ~10^6 cells
-they leave SIMDs without a wave.  us per step, marches -> flat:
-  HLLD  20x20 157 -> 13, 64^3 397 -> 66, 96^3 416 -> 210, 128^3 555 -> 498,
-        160^3 1068 -> 938, 192^3 1515 -> 1562
+HLLD's per-cell part once, but several cells sit in a thread: below ~10^6
+cells they leave SIMDs without a wave.  us per step, marches -> flat:
+  HLLD  48^3 76 -> 36, 64^3 95 -> 65, 96^3 204 -> 204, 112^3 295 -> 330
   HLL   20x20 26 -> 12, 64^3 139 -> 54, 96^3 238 -> 170, 128^3 376 -> 418
   Roe   20x20 33 -> 15, 64^3 101 -> 82, 96^3 328 -> 267, 128^3 605 -> 621
-so HLLD crosses over between 160^3 and 192^3, the others between 96^3 and
-128^3.  Kernel timing keeps the launches it accounts for.
+so all cross over at about 100^3 cells.  Kernel timing keeps the launches it
+accounts for.
 */
-bool flat_step(const pamhd_handle* h, int solver)
+bool flat_step(const pamhd_handle* h)
 {
 	if (h->timing) return false;
-	if (h->tune.flat >= 0) return h->tune.flat == 1;
-	return h->g.n <= (solver == HLLD_ATHENA ? 1ll << 22 : 1ll << 20);
+	return h->tune.flat >= 0 ? h->tune.flat == 1 : h->g.n <= 1ll << 20;
 }
 
 template <class T>
@@ -4415,7 +4481,7 @@ int do_step(pamhd_handle* h, int solver, double max_dt, double cfl, int refits,
 	}
 	StepStatus* prev = h->status + h->last;
 	StepStatus* next = h->status + (1 - h->last);
-	const bool flat = flat_step(h, solver);
+	const bool flat = flat_step(h);
 	if (flat) {
 		const bool report = dt_taken != nullptr;
 		const int e = h->precision == PAMHD_MIXED
@@ -5347,9 +5413,10 @@ int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen, void* 
 		h->tune.fused = 0;
 		float best_ms = time_it(step);
 		report += " passes+update=" + std::to_string(best_ms) + "ms";
-		const int chunks[] = {8, 16, 32};
+		const int chunks[] = {0, 8, 16, 32};
 		for (int mode = 1; mode <= 2; mode++)
 		for (int c : chunks) {
+			if (mode == 1 && c == 0) continue;
 			h->tune = best_t;
 			h->tune.fused = mode;
 			if (mode == 1) h->tune.fused_kc = c;
