@@ -329,7 +329,9 @@ def ensemble_run(nbox, steps, solver="hll-athena", cfl=0.3, seed=2024, imf_steps
     # barriers), from the same start and tile shape
     tiles = {"64x4": 0, "32x8": 1, "16x16": 2}
     with Ensemble(boxes) as e2:
-        e2.set_tile(tiles.get(tune.split("; chosen ")[-1].strip(), 1))
+        shape = tune.split("; chosen ")[-1].strip()
+        if shape in tiles:      # else the default, which autotuning chose
+            e2.set_tile(tiles[shape])
         e2.timestep(solver, 0.0, cfl, stream=stream)
         e2.run(solver, cfl, 2, use_graph=False, stream=stream)
         torch.cuda.synchronize()

@@ -556,7 +556,8 @@ program.)
   check        synchronises; per-box time step of the last step and the
                first physics error
   autotune     picks the fastest tile shape of the cell kernels (64x4, 32x8,
-               16x16) on a copy of the state; set_tile sets it
+               16x16 or the default 256x1, consecutive cells) on a copy of
+               the state; set_tile sets one of the first three
 */
 int pamhd_ensemble_create(int nbox, const pamhd_grid_desc* grids, const pamhd_physics* physics,
 	const pamhd_solar_wind_desc* solar_winds, pamhd_ensemble** out);

@@ -61,6 +61,7 @@ struct BoxDev {
 	long long off;
 	double dx, dy, dz;
 	int gx, gy, blk0;
+	unsigned mx, shx, my, shy;   /* flat index / nx and / ny: (c * m) >> sh */
 	int sw_dim, sw_sg;
 	double sw_rho, sw_m[3], sw_E, sw_B[3];
 	double in_rho, in_m[3], in_E;
@@ -80,7 +81,11 @@ struct CellRef {
 	long long g;
 	int b, pad;
 };
-constexpr Tile TILES[3] = {{64, 4}, {32, 8}, {16, 16}};
+/* the last one: 256 consecutive cells of the box's flat index, so that no
+   lane idles past a row's end (64 x 4 tiles idle half of the lanes of a
+   32-cell box and a quarter of a 48- or 96-cell one); indexes below 2^28 */
+constexpr int T_FLAT = 3;
+constexpr Tile TILES[4] = {{64, 4}, {32, 8}, {16, 16}, {256, 1}};
 
 } // namespace
 
@@ -94,7 +99,7 @@ struct BoxSet {
 	BoxDev* boxes = nullptr;
 	int* blockbox = nullptr;
 	int nblocks = 0;
-	int tile = 0;
+	int tile = T_FLAT;
 	int flux3 = 1;   /* the three flux directions in one launch (box_flux3_kernel) */
 	double* S = nullptr;
 	double* P = nullptr;
@@ -128,6 +133,15 @@ __device__ __forceinline__ bool my_cell(const BoxDev* __restrict__ boxes, const 
 	b = blockbox[tl];
 	const BoxDev& B = boxes[b];
 	const int lb = tl - B.blk0;
+	if constexpr (TX == 256) {
+		const unsigned c = (unsigned)lb * 256 + threadIdx.x;
+		if (c >= (unsigned)B.n) return false;
+		const unsigned t = (unsigned)(((unsigned long long)c * B.mx) >> B.shx);
+		k = (int)(((unsigned long long)t * B.my) >> B.shy);
+		j = (int)t - k * B.ny;
+		i = (int)(c - t * (unsigned)B.nx);
+		return true;
+	}
 	const int tx = lb % B.gx, ty = (lb / B.gx) % B.gy;
 	k = lb / (B.gx * B.gy);
 	i = tx * TX + (int)threadIdx.x;
@@ -1103,8 +1117,18 @@ void launch_stage(BoxSet* s, int solver, hipStream_t st, int stage, BoxStatus* s
 	switch (s->tile) {
 	case 0: launch_all<64, 4>(s, solver, st, stage, stat, chain); break;
 	case 1: launch_all<32, 8>(s, solver, st, stage, stat, chain); break;
+	case T_FLAT: launch_all<256, 1>(s, solver, st, stage, stat, chain); break;
 	default: launch_all<16, 16>(s, solver, st, stage, stat, chain); break;
 	}
+}
+
+/* m and sh of the division by d of indexes below 2^28: sh = 28 + ceil(log2
+   d), m = floor(2^sh / d) + 1 */
+void flat_divisor(unsigned d, unsigned& m, unsigned& sh)
+{
+	sh = 28;
+	while ((1u << (sh - 28)) < d) sh++;
+	m = (unsigned)((1ull << sh) / d) + 1;
 }
 
 /* block -> box table for the current tile shape */
@@ -1117,7 +1141,9 @@ hipError_t build_blocks(BoxSet* s)
 		B.gx = (B.nx + t.tx - 1) / t.tx;
 		B.gy = (B.ny + t.ty - 1) / t.ty;
 		B.blk0 = (int)bb.size();
-		const long long nb = (long long)B.gx * B.gy * B.nz;
+		flat_divisor((unsigned)B.nx, B.mx, B.shx);
+		flat_divisor((unsigned)B.ny, B.my, B.shy);
+		const long long nb = s->tile == T_FLAT ? ((long long)B.n + 255) / 256 : (long long)B.gx * B.gy * B.nz;
 		for (long long q = 0; q < nb; q++) bb.push_back(b);
 	}
 	s->nblocks = (int)bb.size();
@@ -1158,11 +1184,16 @@ long long boxset_faces(const BoxSet* s, int box)
 long long boxset_cells(const BoxSet* s, int box) { return s->host[box].n; }
 int boxset_tile(const BoxSet* s) { return s->tile; }
 
+static int use_tile(BoxSet* s, int tile)
+{
+	s->tile = tile;
+	return build_blocks(s) == hipSuccess ? PAMHD_OK : PAMHD_E_DEVICE;
+}
+
 int boxset_set_tile(BoxSet* s, int tile)
 {
 	if (tile < 0 || tile > 2) return PAMHD_E_ARG;
-	s->tile = tile;
-	return build_blocks(s) == hipSuccess ? PAMHD_OK : PAMHD_E_DEVICE;
+	return use_tile(s, tile);
 }
 
 void boxset_destroy(BoxSet* s)
@@ -1355,6 +1386,8 @@ int boxset_create(BoxSet** out, int nbox, const pamhd_grid_desc* grids, const pa
 		}
 		off += n;
 	}
+	for (const BoxDev& B : s->host)
+		if (B.n >= 1 << 28) s->tile = 0;
 	if ((e = build_blocks(s)) != hipSuccess) return bail(e, "blocks");
 	s->nbnd = (long long)bnd.size();
 	s->ninflow = (long long)inflow.size();
@@ -1507,6 +1540,7 @@ int run_persistent_tile(BoxSet* s, double cfl, long steps, hipStream_t st, std::
 	switch (s->tile) {
 	case 0: return run_persistent<SOLVER, 64, 4>(s, cfl, steps, st, err);
 	case 1: return run_persistent<SOLVER, 32, 8>(s, cfl, steps, st, err);
+	case T_FLAT: return run_persistent<SOLVER, 256, 1>(s, cfl, steps, st, err);
 	default: return run_persistent<SOLVER, 16, 16>(s, cfl, steps, st, err);
 	}
 }
@@ -1612,8 +1646,11 @@ int boxset_autotune(BoxSet* s, int solver, double cfl, int steps, hipStream_t st
 	float best_ms = 1e30f;
 	int rc = PAMHD_OK;
 	report += "tiles:";
-	for (int t = 0; t < 3 && rc == PAMHD_OK; t++) {
-		if (boxset_set_tile(s, t) != PAMHD_OK) {
+	int shapes = 4;
+	for (const BoxDev& B : s->host)
+		if (B.n >= 1 << 28) shapes = 3;
+	for (int t = 0; t < shapes && rc == PAMHD_OK; t++) {
+		if (use_tile(s, t) != PAMHD_OK) {
 			rc = PAMHD_E_DEVICE;
 			break;
 		}
@@ -1635,7 +1672,7 @@ int boxset_autotune(BoxSet* s, int solver, double cfl, int steps, hipStream_t st
 		s->last = last0;
 	}
 	(void)hipStreamSynchronize(st);
-	if (rc == PAMHD_OK) rc = boxset_set_tile(s, best);
+	if (rc == PAMHD_OK) rc = use_tile(s, best);
 	report += "; chosen " + std::to_string(TILES[best].tx) + "x" + std::to_string(TILES[best].ty);
 	(void)hipEventDestroy(a);
 	(void)hipEventDestroy(b);
@@ -1650,6 +1687,7 @@ hipError_t boxset_div_face2volume(BoxSet* s, int box, double* avg)
 	switch (s->tile) {
 	case 0: box_div_kernel<64, 4><<<grid, dim3(64, 4, 1)>>>(s->boxes, s->blockbox, s->N, s->S, s->ctype, box, s->partial); break;
 	case 1: box_div_kernel<32, 8><<<grid, dim3(32, 8, 1)>>>(s->boxes, s->blockbox, s->N, s->S, s->ctype, box, s->partial); break;
+	case T_FLAT: box_div_kernel<256, 1><<<grid, dim3(256, 1, 1)>>>(s->boxes, s->blockbox, s->N, s->S, s->ctype, box, s->partial); break;
 	default: box_div_kernel<16, 16><<<grid, dim3(16, 16, 1)>>>(s->boxes, s->blockbox, s->N, s->S, s->ctype, box, s->partial); break;
 	}
 	hipError_t e = hipGetLastError();

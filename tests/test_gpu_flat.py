@@ -150,3 +150,27 @@ def test_flat_step_replays_in_a_graph(gpu):
             if rep == 1:
                 for _ in range(2):
                     assert a.step("hlld-athena", 1e300, 0.3) == b.step("hlld-athena", 1e300, 0.3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["launches", "graph", "persistent"])
+def test_box_cells_by_flat_index(gpu, mode):
+    """solar-wind boxes with their default blocks of 256 consecutive cells,
+    cells a multiple of a block, a few more and a few less, against the oracle"""
+    from pamhd_amd.swbox import Ensemble
+    from test_gpu_swbox import _test_box
+    boxes = [_test_box(cells=c, seed=3 + q) for q, c in enumerate([(8, 8, 8), (11, 31, 9), (5, 17, 6), (9, 9, 19)])]
+    refs = []
+    for sb in boxes:
+        ob = O.Box(sb)
+        r = ob.init()
+        st, steps, t = ob.run(O.HLL, 0.3, 0.0, 1e30, r, max_steps=5)
+        assert st == 0 and steps == 5
+        refs.append(r)
+    with Ensemble(boxes) as e:
+        e.timestep("hll-athena", 0.0, 0.3)
+        print(mode, flush=True)
+        e.run("hll-athena", 0.3, 5, use_graph=mode == "graph", persistent=mode == "persistent")
+        e.check()
+        for q, r in enumerate(refs):
+            np.testing.assert_array_equal(e.download(q), r, err_msg="box %d" % q)
