@@ -2584,7 +2584,7 @@ __device__ __forceinline__ int cidx(const GridDev& g, int i, int j, int k)
    period, 2: smallest time step / 2^substep-min, 3: largest level, 4: faces
    solved) are spread over SS_SLOTS slots each, a wave's atomic going to the
    slot of its block (a few addresses serialise the 2^18 waves' atomics of
-   a 256^3 grid), and folded by ss_fold_kernel / ss_count_kernel before
+   a 256^3 grid), and folded by ss_fold_kernel / ss_count before
    they are read */
 constexpr int SS_SLOTS = 4096;
 constexpr int SS_FOLD = 256;
@@ -2612,15 +2612,15 @@ __global__ __launch_bounds__(SS_FOLD) void ss_clear_kernel(SubstepDev d)
 
 /* the faces solved over the step: the fifth reduction's slots summed into
    the status record (one block of SS_FOLD threads) */
-__global__ __launch_bounds__(SS_FOLD) void ss_count_kernel(SubstepDev d)
+__device__ __forceinline__ void ss_count(const SubstepDev& d, int tid)
 {
 	__shared__ unsigned long long w[SS_FOLD / 64];
 	unsigned long long v = 0;
-	for (int s = threadIdx.x; s < SS_SLOTS; s += SS_FOLD) v += d.scal[4 * SS_SLOTS + s];
+	for (int s = tid; s < SS_SLOTS; s += SS_FOLD) v += d.scal[4 * SS_SLOTS + s];
 	for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-	if (threadIdx.x % 64 == 0) w[threadIdx.x / 64] = v;
+	if (tid % 64 == 0) w[tid / 64] = v;
 	__syncthreads();
-	if (threadIdx.x == 0) {
+	if (tid == 0) {
 		for (int k = 1; k < SS_FOLD / 64; k++) v += w[k];
 		d.status->flux_calcs = v;
 	}
@@ -2650,38 +2650,45 @@ __global__ __launch_bounds__(SS_FOLD) void ss_fold_kernel(SubstepDev d, int q, i
 	}
 }
 
-/* minimize_timestep, source/mhd/solve.hpp:1927-2014: a cell's limit over its
-   six faces, the smallest over the grid and the smallest of time step /
-   2^substep-min (set_minmax_substepping_period, substepping.hpp:333-342) */
+/* minimize_timestep, source/mhd/solve.hpp:1927-2014: a cell's limit t over its
+   six faces, and t / 2^substep-min */
+__device__ __forceinline__ void ss_cell_ts(const GridDev& g, const SubstepDev& d, double cfl, int i,
+	int j, int k, int c, double& t, double& r)
+{
+	t = r = DBL_MAX;
+	if (!ss_active(d, c)) return;
+	const double len[3] = {g.dx, g.dy, g.dz};
+	const int id[3] = {i, j, k};
+	const int N[3] = {g.nx, g.ny, g.nz};
+	for (int q = 0; q < 3; q++) {
+		/* the faces on the cell's two sides, where the neighbour
+		   exists and is of type >= 0 */
+		int lo[3] = {i, j, k}, hi[3] = {i, j, k};
+		lo[q] = ss_coord(id[q] - 1, N[q], d.per[q]);
+		hi[q] = ss_coord(id[q] + 1, N[q], d.per[q]);
+		const int bl = lo[q] < 0 ? -1 : cidx(g, lo[0], lo[1], lo[2]);
+		const int bh = hi[q] < 0 ? -1 : cidx(g, hi[0], hi[1], hi[2]);
+		if (bl >= 0 && ss_active(d, bl)) {
+			const double v = d.maxv[(long long)q * g.n + c];
+			t = v <= 0 ? 0.0 : smin(cfl * len[q] / v, t);
+		}
+		if (bh >= 0 && ss_active(d, bh)) {
+			const double v = d.maxv[(long long)q * g.n + bh];
+			t = v <= 0 ? 0.0 : smin(cfl * len[q] / v, t);
+		}
+	}
+	r = d.opt ? t / (double)(1 << d.opt[c]) : t;
+}
+
+/* the limits of all cells, their smallest t and r over the grid
+   (set_minmax_substepping_period, substepping.hpp:333-342) */
 __global__ __launch_bounds__(BX * BY) void ss_ts_kernel(GridDev g, SubstepDev d, double cfl)
 {
 	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
 	double t = DBL_MAX, r = DBL_MAX;
 	if (i < g.nx && j < g.ny) {
 		const int c = cidx(g, i, j, k);
-		if (ss_active(d, c)) {
-			const double len[3] = {g.dx, g.dy, g.dz};
-			const int id[3] = {i, j, k};
-			const int N[3] = {g.nx, g.ny, g.nz};
-			for (int q = 0; q < 3; q++) {
-				/* the faces on the cell's two sides, where the neighbour
-				   exists and is of type >= 0 */
-				int lo[3] = {i, j, k}, hi[3] = {i, j, k};
-				lo[q] = ss_coord(id[q] - 1, N[q], d.per[q]);
-				hi[q] = ss_coord(id[q] + 1, N[q], d.per[q]);
-				const int bl = lo[q] < 0 ? -1 : cidx(g, lo[0], lo[1], lo[2]);
-				const int bh = hi[q] < 0 ? -1 : cidx(g, hi[0], hi[1], hi[2]);
-				if (bl >= 0 && ss_active(d, bl)) {
-					const double v = d.maxv[(long long)q * g.n + c];
-					t = v <= 0 ? 0.0 : smin(cfl * len[q] / v, t);
-				}
-				if (bh >= 0 && ss_active(d, bh)) {
-					const double v = d.maxv[(long long)q * g.n + bh];
-					t = v <= 0 ? 0.0 : smin(cfl * len[q] / v, t);
-				}
-			}
-			r = d.opt ? t / (double)(1 << d.opt[c]) : t;
-		}
+		ss_cell_ts(g, d, cfl, i, j, k, c, t, r);
 		d.ts[c] = t;
 	}
 	for (int off = 32; off > 0; off >>= 1) {
@@ -2694,11 +2701,30 @@ __global__ __launch_bounds__(BX * BY) void ss_ts_kernel(GridDev g, SubstepDev d,
 	}
 }
 
-/* set_minmax_substepping_period, source/substepping.hpp:264-399: the
-   substep length and each cell's largest level.  floor(log2 x) is exact
+/* a cell's largest level from its limit t, the smallest limit's substep
+   length ret and the largest step (all_zero: the step is no longer than the
+   smallest limit).  floor(log2 x) is exact
    (ilogb); a non-finite ratio gives level 0.  A cell whose substep-min
    exceeds its level (the reference aborts) or whose level exceeds 30 (its
    int period would overflow) reports PAMHD_E_SUBSTEP. */
+__device__ __forceinline__ int ss_cell_level(const GridDev& g, const SubstepDev& d, double max_dt,
+	double ret, bool all_zero, double t, int c)
+{
+	if (!ss_active(d, c) || all_zero || !(t > 0)) return 0;
+	const double x = smin(t, max_dt) / ret;
+	int step = (__builtin_isfinite(x) && x > 0) ? ilogb(x) : 0;
+	if (step < 0) step = 0;
+	const int cap = d.opt ? d.opt[g.n + c] : d.smax;
+	const int lev = cap > step ? step : cap;
+	if ((d.opt && d.opt[c] > lev) || lev > 30) {
+		record_error(d.status, PAMHD_E_SUBSTEP, c);
+		return 0;
+	}
+	return lev;
+}
+
+/* set_minmax_substepping_period, source/substepping.hpp:264-399: the
+   substep length and each cell's largest level */
 __global__ __launch_bounds__(BX * BY) void ss_level_kernel(GridDev g, SubstepDev d, double max_dt)
 {
 	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
@@ -2709,18 +2735,7 @@ __global__ __launch_bounds__(BX * BY) void ss_level_kernel(GridDev g, SubstepDev
 	int lev = 0;
 	if (i < g.nx && j < g.ny) {
 		const int c = cidx(g, i, j, k);
-		const double t = d.ts[c];
-		if (ss_active(d, c) && !all_zero && t > 0) {
-			const double x = smin(t, max_dt) / ret;
-			int step = (__builtin_isfinite(x) && x > 0) ? ilogb(x) : 0;
-			if (step < 0) step = 0;
-			const int cap = d.opt ? d.opt[g.n + c] : d.smax;
-			lev = cap > step ? step : cap;
-			if ((d.opt && d.opt[c] > lev) || lev > 30) {
-				record_error(d.status, PAMHD_E_SUBSTEP, c);
-				lev = 0;
-			}
-		}
+		lev = ss_cell_level(g, d, max_dt, ret, all_zero, d.ts[c], c);
 		d.e[0][c] = lev;
 	}
 	for (int off = 32; off > 0; off >>= 1) {
@@ -2881,6 +2896,213 @@ __global__ __launch_bounds__(BX * BY) void ss_blockmask_kernel(GridDev g, Subste
 	}
 	/* the list lengths of the first substep (odd) start at zero */
 	if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid < SS_LISTS) d.count[SS_LISTS + tid] = 0;
+}
+
+/*
+The whole preparation of a substepped step (ss_clear_kernel to
+ss_blockmask_kernel with the folds and the restriction's passes between
+them) by one block, for grids of at most SS_PREP_CELLS cells and
+SS_PREP_BLOCKS blocks: those kernels take a few microseconds each however few
+the cells are, and the host has to read the largest level between them to
+know the number of restriction passes.  The same per-cell operations, minima
+and maxima over the cells; the levels that the cells exchange stay in LDS,
+with a block barrier after each pass.  Its time is latency: for the 1002-cell
+shock tube 37 us with the levels in global memory and global atomics for the
+blocks' minima (22 us of it those, waited for at the end), 19 us with LDS for
+both, 9.8 us without the passes that cannot matter when all periods are 1.
+A step of that tube: 9 launches, 4 copies and a host wait less; 175 us
+before, 76 us with this and the merged passes.
+*/
+constexpr int SS_PREP = 1024;
+constexpr int SS_PREP_CELLS = 16 * SS_PREP;
+constexpr int SS_PREP_BLOCKS = 1024;   /* blocks of the cell grid, at most */
+
+__global__ __launch_bounds__(SS_PREP) void ss_prep_kernel(GridDev g, FlatGrid fg, SubstepDev d, double cfl,
+	double max_dt, unsigned long long* host, StepStatus* host_status)
+{
+	/* the cells' levels (two sets for the restriction), P_NONE for a cell
+	   not solved, and the smallest level around each */
+	constexpr signed char P_NONE = 100;
+	__shared__ signed char lev_s[2][SS_PREP_CELLS], low_s[SS_PREP_CELLS];
+	__shared__ int blk_s[4 * SS_PREP_BLOCKS];
+	__shared__ unsigned long long red_t[SS_PREP / 64], red_r[SS_PREP / 64];
+	__shared__ int red_i[SS_PREP / 64];
+	const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+	const int n = (int)g.n;
+	/* the largest v of the block, in every thread */
+	auto block_max = [&](int v) {
+#pragma unroll 1
+		for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
+		__syncthreads();
+		if (lane == 0) red_i[wave] = v;
+		__syncthreads();
+#pragma unroll 1
+		for (int w = 0; w < SS_PREP / 64; w++) v = max(v, red_i[w]);
+		return v;
+	};
+	/* cell c's offset to its neighbour below (s = 0) or above (s = 1) along
+	   a dimension of N cells with the given stride, FAR where there is none */
+	constexpr int FAR = 1 << 30;
+	auto step = [&](int id, int N, int stride, int per, int s) {
+		const bool edge = s ? id + 1 == N : id == 0;
+		const int one = s ? stride : -stride, wrapped = s ? -(N - 1) * stride : (N - 1) * stride;
+		return !edge ? one : per ? wrapped : FAR;
+	};
+	const int sy = g.nx, sz = g.nx * g.ny;
+	/* the smallest level of the 18 face and edge neighbours */
+	auto neighbour_min = [&](const signed char* e, int c) {
+		int i, j, k;
+		fg.cell(g, c, i, j, k);
+		const int xl = step(i, g.nx, 1, d.per[0], 0), xh = step(i, g.nx, 1, d.per[0], 1);
+		const int yl = step(j, g.ny, sy, d.per[1], 0), yh = step(j, g.ny, sy, d.per[1], 1);
+		const int zl = step(k, g.nz, sz, d.per[2], 0), zh = step(k, g.nz, sz, d.per[2], 1);
+		int least = P_NONE;
+#pragma unroll 1
+		for (int q = 0; q < 27; q++) {
+			const int a = q % 3, b = (q / 3) % 3, f = q / 9;
+			const int off = (a != 1) + (b != 1) + (f != 1);
+			if (off == 0 || off == 3) continue;
+			const int x = a == 0 ? xl : a == 1 ? 0 : xh;
+			const int y = b == 0 ? yl : b == 1 ? 0 : yh;
+			const int z = f == 0 ? zl : f == 1 ? 0 : zh;
+			if (x != FAR && y != FAR && z != FAR) least = min(least, (int)e[c + x + y + z]);
+		}
+		return least;
+	};
+	if (tid == 0) {
+		d.status->err = 0;
+		d.status->err_face = -1;
+		d.status->flux_calcs = 0;
+	}
+	for (int s = tid; s < SS_SLOTS; s += SS_PREP) d.scal[4 * SS_SLOTS + s] = 0;
+	for (int b = tid; b < 4 * d.nblk; b += SS_PREP) {
+		blk_s[b] = INT_MAX;
+		if (b < 3 * d.nblk) d.dirty[b] = 1;
+	}
+	if (tid < SS_LISTS) d.count[SS_LISTS + tid] = 0;
+	for (int c = tid; c < n; c += SS_PREP) lev_s[0][c] = ss_active(d, c) ? (signed char)0 : P_NONE;
+	__syncthreads();
+	double t = DBL_MAX, r = DBL_MAX;
+	for (int c = tid; c < n; c += SS_PREP) {
+		int i, j, k;
+		fg.cell(g, c, i, j, k);
+		/* ss_cell_ts, with the types from LDS, the six speeds loaded at once
+		   and one quotient per dimension (the larger speed's is the smaller) */
+		double v[3];
+		bool low = false;
+#pragma unroll
+		for (int q = 0; q < 3; q++) {
+			const int id = q == 0 ? i : q == 1 ? j : k, N = q == 0 ? g.nx : q == 1 ? g.ny : g.nz;
+			const int stride = q == 0 ? 1 : q == 1 ? sy : sz;
+			const int dn = step(id, N, stride, d.per[q], 0), up = step(id, N, stride, d.per[q], 1);
+			const double* mv = d.maxv + (long long)q * g.n;
+			const double a = mv[c], b = mv[up == FAR ? c : c + up];
+			const bool ha = dn != FAR && lev_s[0][dn == FAR ? c : c + dn] != P_NONE;
+			const bool hb = up != FAR && lev_s[0][up == FAR ? c : c + up] != P_NONE;
+			low = low || (ha && a <= 0) || (hb && b <= 0);
+			v[q] = smax(ha ? a : 0.0, hb ? b : 0.0);
+		}
+		double tc = DBL_MAX, rc = DBL_MAX;
+		if (lev_s[0][c] != P_NONE) {
+#pragma unroll
+			for (int q = 0; q < 3; q++)
+				if (v[q] > 0) tc = smin(cfl * (q == 0 ? g.dx : q == 1 ? g.dy : g.dz) / v[q], tc);
+			if (low) tc = 0;
+			rc = d.opt ? tc / (double)(1 << d.opt[c]) : tc;
+		}
+		d.ts[c] = tc;
+		t = smin(t, tc);
+		r = smin(r, rc);
+	}
+#pragma unroll 1
+	for (int off = 32; off > 0; off >>= 1) {
+		t = smin(t, __shfl_xor(t, off, 64));
+		r = smin(r, __shfl_xor(r, off, 64));
+	}
+	/* across waves by the ordered bit patterns, as the atomics of
+	   ss_ts_kernel */
+	if (lane == 0) {
+		red_t[wave] = (unsigned long long)__double_as_longlong(t);
+		red_r[wave] = (unsigned long long)__double_as_longlong(r);
+	}
+	__syncthreads();
+	{
+		unsigned long long tb = (unsigned long long)__double_as_longlong(DBL_MAX), rb = tb;
+#pragma unroll 1
+		for (int w = 0; w < SS_PREP / 64; w++) {
+			tb = red_t[w] < tb ? red_t[w] : tb;
+			rb = red_r[w] < rb ? red_r[w] : rb;
+		}
+		t = __longlong_as_double((long long)tb);
+		r = __longlong_as_double((long long)rb);
+	}
+	const bool all_zero = max_dt <= t;
+	int most = 0;
+	for (int c = tid; c < n; c += SS_PREP) {
+		if (lev_s[0][c] == P_NONE) continue;
+		const int lev = ss_cell_level(g, d, max_dt, r, all_zero, d.ts[c], c);
+		lev_s[0][c] = (signed char)lev;
+		most = max(most, lev);
+	}
+	/* (block_max's barriers end the pass) */
+	const int passes = block_max(most);
+	int cur = 0;
+	for (int q = 0; q < passes; q++) {
+		for (int c = tid; c < n; c += SS_PREP) {
+			int v = lev_s[cur][c];
+			if (v != P_NONE) v = min(v, neighbour_min(lev_s[cur], c) + 1);
+			lev_s[1 - cur][c] = (signed char)v;
+		}
+		__syncthreads();
+		cur = 1 - cur;
+	}
+	const signed char* e = lev_s[cur];
+	int p = 0;
+	for (int c = tid; c < n; c += SS_PREP) {
+		int lev = e[c], low = 0;
+		if (lev == P_NONE) {
+			lev = 0;
+		} else {
+			low = passes > 0 ? min(lev, neighbour_min(e, c)) : lev;   /* (all 0) */
+			p = max(p, 1 << lev);
+		}
+		low_s[c] = (signed char)low;
+		d.period[c] = 1 << lev;
+		d.minsub[c] = 1 << low;
+	}
+	const int largest = block_max(p);
+	/* the blocks' smallest periods, for the lists of the substeps before the
+	   last: none when every period is 1 */
+	if (largest > 1) {
+		const int gx = (g.nx + BX - 1) / BX, gy = (g.ny + BY - 1) / BY;
+		auto period = [&](int c) { return e[c] == P_NONE ? 1 : 1 << e[c]; };
+		for (int c = tid; c < n; c += SS_PREP) {
+			int i, j, k;
+			fg.cell(g, c, i, j, k);
+			const int b = i / BX + gx * (j / BY + gy * k);
+			int least = period(c);
+#pragma unroll 1
+			for (int q = 0; q < 3; q++) {
+				const int dn = q == 0 ? step(i, g.nx, 1, d.per[0], 0) : q == 1 ? step(j, g.ny, sy, d.per[1], 0)
+					: step(k, g.nz, sz, d.per[2], 0);
+				if (dn == FAR) continue;
+				atomicMin(&blk_s[q * d.nblk + b], 1 << low_s[c + dn]);
+				least = min(least, period(c + dn));
+			}
+			atomicMin(&blk_s[3 * d.nblk + b], least);
+		}
+		__syncthreads();
+		for (int b = tid; b < 4 * d.nblk; b += SS_PREP) d.blk[b] = blk_s[b];
+	}
+	if (tid == 0) {
+		const double sub_dt = all_zero ? max_dt : r;
+		*d.sub_dt = sub_dt;
+		host[0] = (unsigned long long)largest;
+		host[1] = (unsigned long long)__double_as_longlong(sub_dt);
+		/* written by atomics and stores of other waves */
+		host_status->err = __hip_atomic_load(&d.status->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		host_status->err_face = __hip_atomic_load(&d.status->err_face, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
 }
 
 /*
@@ -3058,23 +3280,31 @@ __device__ __forceinline__ void ss_flux_block(const GridDev& g, const SubstepDev
 	Em[n + c] = cq[D == 0 ? B0 + 2 : B0];
 }
 
-/* the flux pass of direction D: with WALK over the blocks of its list
-   (those with a face due), else over every block of the cell grid (a
+/* the flux pass of one direction over every block of the cell grid (a
    substep at which every face is due) */
-template <int SOLVER, int D, bool WALK>
+template <int SOLVER, int D>
 __global__ __launch_bounds__(BX * BY) void ss_flux_kernel(GridDev g, SubstepDev d,
 	const double* __restrict__ bg, double* __restrict__ emf, int sub)
 {
-	if constexpr (WALK) {
-		const int cnt = d.count[SS_LISTS * (sub & 1) + D];
-		const int* list = d.list + (size_t)D * d.nblk;
-		for (int idx = blockIdx.x; idx < cnt; idx += gridDim.x) {
-			int bx, by, bz;
-			ss_block_coords(g, list[idx], bx, by, bz);
-			ss_flux_block<SOLVER, D>(g, d, bg, emf, sub, bx, by, bz);
-		}
-	} else {
-		ss_flux_block<SOLVER, D>(g, d, bg, emf, sub, blockIdx.x, blockIdx.y, blockIdx.z);
+	ss_flux_block<SOLVER, D>(g, d, bg, emf, sub, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+/* the flux passes of the three directions in one launch, direction
+   blockIdx.y: with WALK over the blocks of each direction's list (those
+   with a face due), else over every block, blockIdx.x their index */
+template <int SOLVER, bool WALK>
+__global__ __launch_bounds__(BX * BY) void ss_flux3_kernel(GridDev g, SubstepDev d,
+	const double* __restrict__ bg, double* __restrict__ emf, int sub)
+{
+	const int D = (int)blockIdx.y;
+	const int cnt = WALK ? d.count[SS_LISTS * (sub & 1) + D] : d.nblk;
+	const int* list = d.list + (size_t)D * d.nblk;
+	for (int idx = blockIdx.x; idx < cnt; idx += gridDim.x) {
+		int bx, by, bz;
+		ss_block_coords(g, WALK ? list[idx] : idx, bx, by, bz);
+		if (D == 0) ss_flux_block<SOLVER, 0>(g, d, bg, emf, sub, bx, by, bz);
+		else if (D == 1) ss_flux_block<SOLVER, 1>(g, d, bg, emf, sub, bx, by, bz);
+		else ss_flux_block<SOLVER, 2>(g, d, bg, emf, sub, bx, by, bz);
 	}
 }
 
@@ -3180,13 +3410,13 @@ __global__ __launch_bounds__(BX * BY) void ss_flux_march_kernel(GridDev g, Subst
 		atomicAdd(&d.scal[4 * SS_SLOTS + ss_slot()], (unsigned long long)solved);
 }
 
-/* the edge fields of direction D set to zero in the blocks of its zeroing
-   list (no face due, the previous substep's values still there), what the
-   flux pass would write there */
-template <int D>
+/* the edge fields of direction D (blockIdx.y) set to zero in the blocks of
+   its zeroing list (no face due, the previous substep's values still
+   there), what the flux pass would write there */
 __global__ __launch_bounds__(BX * BY) void ss_zero_emf_kernel(GridDev g, SubstepDev d,
 	double* __restrict__ emf, int sub)
 {
+	const int D = (int)blockIdx.y;
 	const int cnt = d.count[SS_LISTS * (sub & 1) + SS_LIST_ZERO + D];
 	const int* list = d.list + (size_t)(SS_LIST_ZERO + D) * d.nblk;
 	const long long n = g.n;
@@ -3269,21 +3499,24 @@ __device__ __forceinline__ void ss_dbsum_block(const GridDev& g, const SubstepDe
 }
 
 /* the face-dB pass, with WALK over the blocks of its list (those around
-   which a face is due) and, with ZERO_DB, of its list of blocks with a sum
-   that restarts and no face due around them (a block with neither is in
-   no list: every dB is +0 and no sum changes); else over every block */
-template <bool WALK, bool ZERO_DB>
+   which a face is due; blockIdx.y 1) and of its list of blocks with a sum
+   that restarts and no face due around them (blockIdx.y 0; a block with
+   neither is in no list: every dB is +0 and no sum changes); else over
+   every block */
+template <bool WALK>
 __global__ __launch_bounds__(BX * BY) void ss_dbsum_kernel(GridDev g, SubstepDev d,
 	const double* __restrict__ emf, int sub)
 {
 	if constexpr (WALK) {
-		const int l = ZERO_DB ? SS_LIST_DB0 : SS_LIST_DB;
+		const bool zero = blockIdx.y == 0;
+		const int l = zero ? SS_LIST_DB0 : SS_LIST_DB;
 		const int cnt = d.count[SS_LISTS * (sub & 1) + l];
 		const int* list = d.list + (size_t)l * d.nblk;
 		for (int idx = blockIdx.x; idx < cnt; idx += gridDim.x) {
 			int bx, by, bz;
 			ss_block_coords(g, list[idx], bx, by, bz);
-			ss_dbsum_block<ZERO_DB>(g, d, emf, sub, bx, by, bz);
+			if (zero) ss_dbsum_block<true>(g, d, emf, sub, bx, by, bz);
+			else ss_dbsum_block<false>(g, d, emf, sub, bx, by, bz);
 		}
 	} else {
 		ss_dbsum_block<false>(g, d, emf, sub, blockIdx.x, blockIdx.y, blockIdx.z);
@@ -3396,13 +3629,25 @@ __global__ __launch_bounds__(BX * BY) void ss_update_kernel(GridDev g, SubstepDe
 	}
 }
 
+/* what the host reads after a step: the error and the faces solved */
+__device__ __forceinline__ void ss_report(const StepStatus* st, StepStatus* host)
+{
+	host->err = st->err;
+	host->err_face = st->err_face;
+	host->flux_calcs = st->flux_calcs;
+}
+
+__global__ __launch_bounds__(SS_FOLD) void ss_end_kernel(SubstepDev d, int count, StepStatus* host)
+{
+	if (count) ss_count(d, threadIdx.x);
+	if (threadIdx.x == 0) ss_report(d.status, host);
+}
+
 /* sync_magnetic_field, common_functions.hpp:184-269: the two visits to a
    face, the cell with the smaller index first */
 template <int D>
-__global__ __launch_bounds__(BX * BY) void ss_sync_kernel(GridDev g, SubstepDev d)
+__device__ __forceinline__ void ss_sync_face(const GridDev& g, const SubstepDev& d, int i, int j, int k)
 {
-	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
-	if (i >= g.nx || j >= g.ny) return;
 	const long long n = g.n;
 	const int b = cidx(g, i, j, k);
 	const int ai = D == 0 ? ss_coord(i - 1, g.nx, d.per[0]) : i;
@@ -3425,6 +3670,22 @@ __global__ __launch_bounds__(BX * BY) void ss_sync_kernel(GridDev g, SubstepDev 
 	d.S[(8 + 2 * D) * n + b] = pb;
 }
 
+/* the faces on each cell's negative sides (a face's two copies belong to
+   no other face); the plane of blocks past the grid, where there is one,
+   reports to the host */
+__global__ __launch_bounds__(BX * BY) void ss_sync_kernel(GridDev g, SubstepDev d, StepStatus* host)
+{
+	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
+	if (k == g.nz) {
+		if (i == 0 && j == 0) ss_report(d.status, host);
+		return;
+	}
+	if (i >= g.nx || j >= g.ny) return;
+	ss_sync_face<0>(g, d, i, j, k);
+	ss_sync_face<1>(g, d, i, j, k);
+	ss_sync_face<2>(g, d, i, j, k);
+}
+
 /* update_vol_B(0) of all cells and the face-once state; with `refit`
    also the constant-pressure refit of the main loop's apply_boundaries
    (refit_kernel's, with the field of the face-once state: the cell's and
@@ -3433,9 +3694,19 @@ __global__ __launch_bounds__(BX * BY) void ss_sync_kernel(GridDev g, SubstepDev 
    state written here (energy, face-average field, +d copies from the
    neighbours' -d copies), so the next step may skip that expansion */
 __global__ __launch_bounds__(BX * BY) void ss_final_kernel(GridDev g, SubstepDev d, double* __restrict__ s,
-	int refit)
+	int refit, StepStatus* host)
 {
+	static_assert(SS_FOLD == BX * BY, "the counting block");
 	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
+	/* the first block of the plane past the grid counts the faces solved
+	   and reports to the host */
+	if (k == g.nz) {
+		if (blockIdx.x == 0 && blockIdx.y == 0) {
+			ss_count(d, threadIdx.x + BX * threadIdx.y);
+			if (threadIdx.x == 0 && threadIdx.y == 0) ss_report(d.status, host);
+		}
+		return;
+	}
 	if (i >= g.nx || j >= g.ny) return;
 	const long long n = g.n;
 	const int c = cidx(g, i, j, k);
@@ -4020,10 +4291,11 @@ apply_boundaries on a grid with boundaries (source/mhd/boundaries.hpp:
 1261-1297): value and copy boundaries of number density, velocity and
 pressure (apply_fluid_boundaries, :738-1026), of the face field
 (apply_magnetic_field_boundaries_staggered, :250-640, uniform grids), then
-update_vol_B(0) at constant pressure of every cell of type >= 0.  One
-launch per stage; a stage writes only boundary cells and reads only its
-own cell and normal cells, which no stage writes.  Neighbours are visited
-in the order of the neighbourhood (offsets -1..1, z slowest).
+update_vol_B(0) at constant pressure of every cell of type >= 0.  A stage
+before that writes only boundary cells and reads only its own cell and
+normal cells, which none of them writes, so a thread takes its cell through
+all of them (bnd_apply_kernel).  Neighbours are visited in the order of the
+neighbourhood (offsets -1..1, z slowest).
 */
 struct BndNb { int id; int fn; int en0, en1, en2; };
 
@@ -4074,10 +4346,9 @@ __device__ __forceinline__ double bnd_pressure(const SubstepDev& d, long long n,
 
 /* STAGE 0 number density, 1 velocity, 2 pressure */
 template <int STAGE>
-__global__ __launch_bounds__(BX * BY) void bnd_fluid_kernel(GridDev g, SubstepDev d, double proton_mass)
+__device__ __forceinline__ void bnd_fluid(const GridDev& g, const SubstepDev& d, double proton_mass, int i,
+	int j, int k)
 {
-	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
-	if (i >= g.nx || j >= g.ny) return;
 	const long long n = g.n;
 	const int c = cidx(g, i, j, k);
 	if (d.bmask[STAGE * n + c]) {
@@ -4139,10 +4410,8 @@ __global__ __launch_bounds__(BX * BY) void bnd_fluid_kernel(GridDev g, SubstepDe
 	}
 }
 
-__global__ __launch_bounds__(BX * BY) void bnd_field_value_kernel(GridDev g, SubstepDev d)
+__device__ __forceinline__ void bnd_field_value(const GridDev& g, const SubstepDev& d, int i, int j, int k)
 {
-	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
-	if (i >= g.nx || j >= g.ny) return;
 	const long long n = g.n;
 	const int c = cidx(g, i, j, k);
 	if (!d.bmask[3 * n + c]) return;
@@ -4151,10 +4420,8 @@ __global__ __launch_bounds__(BX * BY) void bnd_field_value_kernel(GridDev g, Sub
 	}
 }
 
-__global__ __launch_bounds__(BX * BY) void bnd_field_copy_kernel(GridDev g, SubstepDev d)
+__device__ __forceinline__ void bnd_field_copy(const GridDev& g, const SubstepDev& d, int i, int j, int k)
 {
-	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
-	if (i >= g.nx || j >= g.ny) return;
 	const long long n = g.n;
 	const int c = cidx(g, i, j, k);
 	if (d.vt[3 * n + c] != 4) return;
@@ -4195,6 +4462,20 @@ __global__ __launch_bounds__(BX * BY) void bnd_field_copy_kernel(GridDev g, Subs
 		}
 		d.S[(8 + f) * n + c] = F[f];
 	}
+}
+
+/* the stages of one cell in order: each writes only its own cell (a boundary
+   cell; its faces of type 1 with the values they have) and reads that cell
+   and what no stage changes (normal cells, faces of type 1) */
+__global__ __launch_bounds__(BX * BY) void bnd_apply_kernel(GridDev g, SubstepDev d, double proton_mass)
+{
+	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
+	if (i >= g.nx || j >= g.ny) return;
+	bnd_fluid<0>(g, d, proton_mass, i, j, k);
+	bnd_fluid<1>(g, d, proton_mass, i, j, k);
+	bnd_fluid<2>(g, d, proton_mass, i, j, k);
+	bnd_field_value(g, d, i, j, k);
+	bnd_field_copy(g, d, i, j, k);
 }
 
 /* update_vol_B(0) with constant pressure of the cells of type >= 0 */
@@ -4303,15 +4584,21 @@ dim3 ss_walk_grid(const SubstepDev& d)
 }
 
 /* the flux passes of substep `sub`; at a substep where every face is due
-   (full) they cover the whole cell grid, and no edge field needs zeroing */
+   (full) they cover the whole cell grid, and no edge field needs zeroing.
+   Up to 2^20 cells the three directions share a launch (per face: marches
+   leave the GPU idle there, as in flat_step) */
 template <int SOLVER>
 void ss_launch_flux(pamhd_handle* h, double* P, int sub, bool full, hipStream_t st)
 {
 	const SubstepDev& d = *h->sub;
 	const dim3 block(BX, BY, 1);
 	if (full) {
+		if (h->g.n <= 1ll << 20) {
+			ss_flux3_kernel<SOLVER, false><<<dim3((unsigned)d.nblk, 3, 1), block, 0, st>>>(h->g, d, h->bg, P, sub);
+			return;
+		}
 		const dim3 grid = cell_grid(h->g);
-		ss_flux_kernel<SOLVER, 0, false><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
+		ss_flux_kernel<SOLVER, 0><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
 		if constexpr (SOLVER == HLLD_ATHENA) {
 			if (!d.bounded && !d.ct) {
 				/* HLLD's per-cell part carried along marches of 16 cells */
@@ -4324,35 +4611,41 @@ void ss_launch_flux(pamhd_handle* h, double* P, int sub, bool full, hipStream_t 
 				return;
 			}
 		}
-		ss_flux_kernel<SOLVER, 1, false><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
-		ss_flux_kernel<SOLVER, 2, false><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
+		ss_flux_kernel<SOLVER, 1><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
+		ss_flux_kernel<SOLVER, 2><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
 		return;
 	}
-	const dim3 grid = ss_walk_grid(d);
-	ss_zero_emf_kernel<0><<<grid, block, 0, st>>>(h->g, d, P, sub);
-	ss_zero_emf_kernel<1><<<grid, block, 0, st>>>(h->g, d, P, sub);
-	ss_zero_emf_kernel<2><<<grid, block, 0, st>>>(h->g, d, P, sub);
-	ss_flux_kernel<SOLVER, 0, true><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
-	ss_flux_kernel<SOLVER, 1, true><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
-	ss_flux_kernel<SOLVER, 2, true><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
+	const dim3 grid(ss_walk_grid(d).x, 3, 1);
+	ss_zero_emf_kernel<<<grid, block, 0, st>>>(h->g, d, P, sub);
+	ss_flux3_kernel<SOLVER, true><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
+}
+
+/* the grid of a kernel over the cells with a plane of blocks past them,
+   where a launch can have one more (else ss_end runs on its own) */
+constexpr unsigned GRID_Z_MOST = 65535;
+dim3 cell_grid_and_plane(const GridDev& g)
+{
+	dim3 d = cell_grid(g);
+	if (d.z < GRID_Z_MOST) d.z++;
+	return d;
+}
+
+void ss_end(pamhd_handle* h, bool count, hipStream_t st)
+{
+	if (cell_grid(h->g).z >= GRID_Z_MOST)
+		ss_end_kernel<<<1, SS_FOLD, 0, st>>>(*h->sub, count ? 1 : 0, h->sub->host_status);
 }
 
 /* apply_boundaries and the main loop's sync_magnetic_field on a grid with
-   boundaries */
+   boundaries; the last launch reports to the host */
 void launch_boundaries(pamhd_handle* h, hipStream_t st)
 {
 	SubstepDev& d = *h->sub;
 	const dim3 grid = cell_grid(h->g), block(BX, BY, 1);
-	const double mp = h->phys.proton_mass;
-	bnd_fluid_kernel<0><<<grid, block, 0, st>>>(h->g, d, mp);
-	bnd_fluid_kernel<1><<<grid, block, 0, st>>>(h->g, d, mp);
-	bnd_fluid_kernel<2><<<grid, block, 0, st>>>(h->g, d, mp);
-	bnd_field_value_kernel<<<grid, block, 0, st>>>(h->g, d);
-	bnd_field_copy_kernel<<<grid, block, 0, st>>>(h->g, d);
+	bnd_apply_kernel<<<grid, block, 0, st>>>(h->g, d, h->phys.proton_mass);
 	bnd_refit_kernel<<<grid, block, 0, st>>>(h->g, d);
-	ss_sync_kernel<0><<<grid, block, 0, st>>>(h->g, d);
-	ss_sync_kernel<1><<<grid, block, 0, st>>>(h->g, d);
-	ss_sync_kernel<2><<<grid, block, 0, st>>>(h->g, d);
+	ss_sync_kernel<<<cell_grid_and_plane(h->g), block, 0, st>>>(h->g, d, d.host_status);
+	ss_end(h, false, st);
 }
 
 /* timestep() with per-cell substepping (and apply_boundaries' refit when
@@ -4363,33 +4656,40 @@ int substep_step(pamhd_handle* h, int solver, double max_dt, double cfl, int ref
 	SubstepDev& d = *h->sub;
 	const dim3 grid = cell_grid(h->g), block(BX, BY, 1);
 	double* P = h->flux;   /* the substep's field components per face, 6 x n (of 24 x n) */
-	ss_clear_kernel<<<1, SS_FOLD, 0, st>>>(d);
-	ss_ts_kernel<<<grid, block, 0, st>>>(h->g, d, cfl);
-	ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 0, 1);
-	ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 2, 1);
-	ss_level_kernel<<<grid, block, 0, st>>>(h->g, d, max_dt);
-	ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 3, 0);
-	HIP_TRY(h, hipGetLastError());
-	HIP_TRY(h, hipMemcpyAsync(d.host + 2, d.scal + 3 * SS_SLOTS, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-	HIP_TRY(h, hipMemcpyAsync(d.host_status, d.status, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
-	HIP_TRY(h, hipStreamSynchronize(st));
-	if (d.host_status->err) return report_status(h, *d.host_status);
-	/* Jacobi passes of the restriction: a cell's restricted level is the
-	   smallest over cells m of level(m) + distance, reached within as many
-	   passes as the largest level */
-	const int passes = (int)d.host[2];
-	int cur = 0;
-	for (int r = 0; r < passes; r++) {
-		ss_restrict_kernel<<<grid, block, 0, st>>>(h->g, d, d.e[cur], d.e[1 - cur]);
-		cur = 1 - cur;
+	if (h->g.n <= SS_PREP_CELLS && d.nblk <= SS_PREP_BLOCKS) {
+		ss_prep_kernel<<<1, SS_PREP, 0, st>>>(h->g, FlatGrid{flat_div((unsigned)h->g.nx), flat_div((unsigned)h->g.ny)}, d, cfl, max_dt, d.host, d.host_status);
+		HIP_TRY(h, hipGetLastError());
+		HIP_TRY(h, hipStreamSynchronize(st));
+		if (d.host_status->err) return report_status(h, *d.host_status);
+	} else {
+		ss_clear_kernel<<<1, SS_FOLD, 0, st>>>(d);
+		ss_ts_kernel<<<grid, block, 0, st>>>(h->g, d, cfl);
+		ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 0, 1);
+		ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 2, 1);
+		ss_level_kernel<<<grid, block, 0, st>>>(h->g, d, max_dt);
+		ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 3, 0);
+		HIP_TRY(h, hipGetLastError());
+		HIP_TRY(h, hipMemcpyAsync(d.host + 2, d.scal + 3 * SS_SLOTS, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+		HIP_TRY(h, hipMemcpyAsync(d.host_status, d.status, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
+		HIP_TRY(h, hipStreamSynchronize(st));
+		if (d.host_status->err) return report_status(h, *d.host_status);
+		/* Jacobi passes of the restriction: a cell's restricted level is the
+		   smallest over cells m of level(m) + distance, reached within as many
+		   passes as the largest level */
+		const int passes = (int)d.host[2];
+		int cur = 0;
+		for (int r = 0; r < passes; r++) {
+			ss_restrict_kernel<<<grid, block, 0, st>>>(h->g, d, d.e[cur], d.e[1 - cur]);
+			cur = 1 - cur;
+		}
+		ss_period_kernel<<<grid, block, 0, st>>>(h->g, d, d.e[cur]);
+		ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 1, 0);
+		ss_blockmask_kernel<<<grid, block, 0, st>>>(h->g, d);
+		HIP_TRY(h, hipGetLastError());
+		HIP_TRY(h, hipMemcpyAsync(d.host, d.scal + 1 * SS_SLOTS, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+		HIP_TRY(h, hipMemcpyAsync(d.host + 1, d.sub_dt, sizeof(double), hipMemcpyDeviceToHost, st));
+		HIP_TRY(h, hipStreamSynchronize(st));
 	}
-	ss_period_kernel<<<grid, block, 0, st>>>(h->g, d, d.e[cur]);
-	ss_fold_kernel<<<1, SS_FOLD, 0, st>>>(d, 1, 0);
-	ss_blockmask_kernel<<<grid, block, 0, st>>>(h->g, d);
-	HIP_TRY(h, hipGetLastError());
-	HIP_TRY(h, hipMemcpyAsync(d.host, d.scal + 1 * SS_SLOTS, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-	HIP_TRY(h, hipMemcpyAsync(d.host + 1, d.sub_dt, sizeof(double), hipMemcpyDeviceToHost, st));
-	HIP_TRY(h, hipStreamSynchronize(st));
 	const int maxp = (int)d.host[0];
 	double sub_dt;
 	memcpy(&sub_dt, d.host + 1, sizeof(double));
@@ -4408,7 +4708,7 @@ int substep_step(pamhd_handle* h, int solver, double max_dt, double cfl, int ref
 		   of two up to maxp): its passes cover the whole grid; the others
 		   walk their lists */
 		const bool full = sub == maxp;
-		ss_lists_kernel<<<(unsigned)((d.nblk + 255) / 256), 256, 0, st>>>(h->g, d, sub);
+		if (!full) ss_lists_kernel<<<(unsigned)((d.nblk + 255) / 256), 256, 0, st>>>(h->g, d, sub);
 		switch (solver) {
 		case RUSANOV: ss_launch_flux<RUSANOV>(h, P, sub, full, st); break;
 		case HLL_ATHENA: ss_launch_flux<HLL_ATHENA>(h, P, sub, full, st); break;
@@ -4417,28 +4717,25 @@ int substep_step(pamhd_handle* h, int solver, double max_dt, double cfl, int ref
 		default: return fail(h, PAMHD_E_SOLVER, "invalid solver " + std::to_string(solver));
 		}
 		if (full) {
-			ss_dbsum_kernel<false, false><<<grid, block, 0, st>>>(h->g, d, P, sub);
+			ss_dbsum_kernel<false><<<grid, block, 0, st>>>(h->g, d, P, sub);
 		} else {
-			ss_dbsum_kernel<true, true><<<ss_walk_grid(d), block, 0, st>>>(h->g, d, P, sub);
-			ss_dbsum_kernel<true, false><<<ss_walk_grid(d), block, 0, st>>>(h->g, d, P, sub);
+			ss_dbsum_kernel<true><<<dim3(ss_walk_grid(d).x, 2, 1), block, 0, st>>>(h->g, d, P, sub);
 		}
 		if (full) ss_update_kernel<false><<<grid, block, 0, st>>>(h->g, d, sub);
 		else ss_update_kernel<true><<<ss_walk_grid(d), block, 0, st>>>(h->g, d, sub);
 	}
-	ss_sync_kernel<0><<<grid, block, 0, st>>>(h->g, d);
-	ss_sync_kernel<1><<<grid, block, 0, st>>>(h->g, d);
-	ss_sync_kernel<2><<<grid, block, 0, st>>>(h->g, d);
+	ss_sync_kernel<<<grid, block, 0, st>>>(h->g, d, nullptr);
 	/* on a periodic grid the final kernel also does apply_boundaries'
-	   refit (refits == 3) */
-	ss_final_kernel<<<grid, block, 0, st>>>(h->g, d, h->state[h->cur], !d.bounded && refits == 3);
+	   refit (refits == 3); the last launch of the step reports to the host */
+	ss_final_kernel<<<cell_grid_and_plane(h->g), block, 0, st>>>(h->g, d, h->state[h->cur],
+		!d.bounded && refits == 3, d.host_status);
+	ss_end(h, true, st);
 	if (!d.bounded) {
 		h->ss_valid = true;
 		h->ss_at = h->calls;
 	}
-	ss_count_kernel<<<1, SS_FOLD, 0, st>>>(d);
 	if (refits == 3 && d.bounded) launch_boundaries(h, st);
 	HIP_TRY(h, hipGetLastError());
-	HIP_TRY(h, hipMemcpyAsync(d.host_status, d.status, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
 	HIP_TRY(h, hipStreamSynchronize(st));
 	d.last_max = maxp;
 	h->flux_calcs = d.host_status->flux_calcs;
@@ -4823,7 +5120,6 @@ int pamhd_apply_boundaries(pamhd_handle* h, double /*simulation_time*/, void* st
 		ss_clear_kernel<<<1, SS_FOLD, 0, st>>>(*h->sub);
 		launch_boundaries(h, st);
 		HIP_TRY(h, hipGetLastError());
-		HIP_TRY(h, hipMemcpyAsync(h->sub->host_status, h->sub->status, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
 		HIP_TRY(h, hipStreamSynchronize(st));
 		return report_status(h, *h->sub->host_status);
 	}

@@ -174,3 +174,25 @@ def test_box_cells_by_flat_index(gpu, mode):
         e.check()
         for q, r in enumerate(refs):
             np.testing.assert_array_equal(e.download(q), r, err_msg="box %d" % q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cells", [(2, 3, 900), (2, 3, 1200), (65, 5, 4), (1, 1, 65535), (32, 32, 17)])
+def test_substep_preparation_paths(gpu, cells):
+    """substepped steps of grids around the limits of the one-block
+    preparation (16384 cells, 1024 blocks of 64 x 4 cells) and with the most
+    planes a launch has (no plane of blocks past them), against the oracle"""
+    from pamhd_amd import configs
+    from pamhd_amd import solver as S
+    state, length, gamma, mu0 = configs.hot_blob(cells, contrast=30.0, radius=0.3, seed=3)
+    ref = state.copy()
+    og = O.make_grid(cells, length, gamma, mu0)
+    st, steps, t, largest = O.run_periodic_substep(og, O.HLLD, 0.3, 0, 999, 0.0, 1e9, ref, max_steps=3)
+    assert st == 0 and largest == 4
+    with S.Grid(cells, length, gamma, mu0) as g:
+        g.upload(state)
+        g.set_substepping(0, 999)
+        print("cells", cells, flush=True)
+        assert g.run("hlld-athena", 0.3, 0.0, 1e9, max_steps=3) == (steps, t)
+        assert g.last_max_substep() == largest
+        np.testing.assert_array_equal(g.download(), ref)
