@@ -108,3 +108,29 @@ def test_clean_divergence_reports_unconverged(gpu):
         assert g.div_face2volume() < d0
         with pytest.raises(_lib.PamhdError):
             g.clean_divergence(tol=1e-14, max_cycles=1)
+
+
+# sizes around the tiles of the residual norm (64 x 4 cells, 8 planes) and of
+# the bottom levels swept by one wave or one block; fields and spacings at
+# which the quotients by a level's constants leave the range of their quick
+# form in some cells, in all, or because of the constant
+@pytest.mark.parametrize("cells,field,spacing", [
+    ((64, 64, 64), 1.0, 1.0), ((66, 6, 10), 1.0, 1.0), ((130, 36, 18), 1.0, 1.0),
+    ((32, 8, 8), 1.0, 1.0), ((8, 8, 4), 1.0, 1.0), ((16, 12, 9), 1.0, 1.0),
+    ((40, 20, 12), 1e-148, 1.0), ((40, 20, 12), 1e-150, 1.0), ((40, 20, 12), 1e100, 1.0),
+    ((40, 20, 12), 1.0, 1e40)])
+def test_clean_divergence_tiles_and_ranges(gpu, cells, field, spacing):
+    from pamhd_amd import solver as S
+    state, length, gamma, mu0 = _perturbed(cells)
+    state = state.copy()
+    state[5:] *= field
+    length = tuple(x * spacing for x in length)
+    st_o, rel_o, cyc_o, ref, og = _oracle_clean(cells, length, gamma, mu0, state, 1e-10)
+    with S.Grid(cells, length, gamma, mu0) as g:
+        g.upload(state)
+        before, rel_g, cyc_g, st_g = g.clean_divergence(tol=1e-10, max_cycles=50, check=False)
+        out = g.download()
+    print(cells, field, spacing, "oracle", st_o, rel_o, cyc_o, "gpu", st_g, rel_g, cyc_g, flush=True)
+    assert cyc_g == cyc_o > 0
+    assert (st_g == 0) == (st_o == 0)
+    np.testing.assert_array_equal(out, ref)
