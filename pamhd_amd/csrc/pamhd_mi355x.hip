@@ -3319,7 +3319,7 @@ into the substep's sums and edge fields as in ss_flux_block.  Blocks: x
 tiles fastest, then BY-line groups, then chunks of km along D.
 */
 template <int D>
-__global__ __launch_bounds__(BX * BY) void ss_flux_march_kernel(GridDev g, SubstepDev d,
+__global__ __launch_bounds__(BX * BY, 3) void ss_flux_march_kernel(GridDev g, SubstepDev d,
 	double* __restrict__ emf, int sub, unsigned gx, int km)
 {
 	static_assert(D == 1 || D == 2, "march along y or z");
@@ -3367,6 +3367,9 @@ __global__ __launch_bounds__(BX * BY) void ss_flux_march_kernel(GridDev g, Subst
 				load(c, U);
 				stage_r = hlld_side<double>(U, g.ph, Rs, cfr, code_r);
 			}
+			/* ahead of the face, whose evaluation covers their latency */
+			const int m = d.minsub[o];
+			const int po = d.period[o], pc = d.period[c];
 			double F[8], sT = 0;
 			int e;
 			if (stage_l | stage_r) e = first_side_error(stage_l, code_l, stage_r, code_r);
@@ -3382,11 +3385,9 @@ __global__ __launch_bounds__(BX * BY) void ss_flux_march_kernel(GridDev g, Subst
 				Fg[M0 + D] = F[M0]; Fg[M0 + (D + 1) % 3] = F[M1]; Fg[M0 + (D + 2) % 3] = F[M2];
 				Fg[B0 + D] = F[B0]; Fg[B0 + (D + 1) % 3] = F[B1]; Fg[B0 + (D + 2) % 3] = F[B2];
 			}
-			const int m = d.minsub[o];
 			const double min_dt = *d.sub_dt * m;
 			double cq[8];
 			for (int q = 0; q < 8; q++) cq[q] = min_dt * Fg[q];
-			const int po = d.period[o], pc = d.period[c];
 			const int pmax = po > pc ? po : pc, pmin = po > pc ? pc : po;
 			const bool fresh = ((sub - m) & (pmax - 1)) == 0;
 			for (int q = 0; q < 8; q++) A[q * n + c] = (fresh ? 0.0 : A[q * n + c]) + cq[q];
@@ -4600,14 +4601,17 @@ void ss_launch_flux(pamhd_handle* h, double* P, int sub, bool full, hipStream_t 
 		const dim3 grid = cell_grid(h->g);
 		ss_flux_kernel<SOLVER, 0><<<grid, block, 0, st>>>(h->g, d, h->bg, P, sub);
 		if constexpr (SOLVER == HLLD_ATHENA) {
-			if (!d.bounded && !d.ct) {
-				/* HLLD's per-cell part carried along marches of 16 cells */
-				const int km = 16;
+			if (!d.bounded && !d.ct && h->g.n > 1ll << 23) {
+				/* HLLD's per-cell part carried along marches, 3 blocks on
+				   a CU: worth it where the marches fill several rounds of
+				   the chip (a step of 256^3 cells 8.87 ms, per face 8.98;
+				   of 200 x 90 x 130 cells 1.85 ms, per face 1.75; a y pass
+				   of 128 x 160 x 192 cells 286 us, per face 252) */
 				const unsigned gx = (h->g.nx + BX - 1) / BX;
-				const unsigned g1 = gx * ((h->g.nz + BY - 1) / BY) * ((h->g.ny + km - 1) / km);
-				const unsigned g2 = gx * ((h->g.ny + BY - 1) / BY) * ((h->g.nz + km - 1) / km);
-				ss_flux_march_kernel<1><<<g1, block, 0, st>>>(h->g, d, P, sub, gx, km);
-				ss_flux_march_kernel<2><<<g2, block, 0, st>>>(h->g, d, P, sub, gx, km);
+				const unsigned gy = gx * ((h->g.nz + BY - 1) / BY), gz = gx * ((h->g.ny + BY - 1) / BY);
+				const int ky = march_cells(gy, h->g.ny, 3, ACC_KMAX), kz = march_cells(gz, h->g.nz, 3, ACC_KMAX);
+				ss_flux_march_kernel<1><<<gy * ((h->g.ny + ky - 1) / ky), block, 0, st>>>(h->g, d, P, sub, gx, ky);
+				ss_flux_march_kernel<2><<<gz * ((h->g.nz + kz - 1) / kz), block, 0, st>>>(h->g, d, P, sub, gx, kz);
 				return;
 			}
 		}

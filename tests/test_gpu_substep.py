@@ -234,3 +234,25 @@ def test_substep_min_above_the_allowed_level_fails_the_step(gpu):
         with pytest.raises(_lib.PamhdError) as e:
             g.step("hll-athena", 1e9, 0.3)
         assert e.value.code == _lib.PAMHD_E_SUBSTEP
+
+
+@pytest.mark.parametrize("repeat", [(2, 2, 2), (4, 4, 4)])
+def test_full_passes_of_large_grids(gpu, repeat):
+    """A grid made of copies of a small periodic one steps as copies of it:
+    above 2^20 cells the passes over every face are a launch per direction,
+    above 2^23 HLLD's y- and z-faces go by marches; the small grid takes
+    neither."""
+    from pamhd_amd.solver import Grid
+    cells = (64, 64, 33)
+    state, length, gamma, mu0 = configs.hot_blob(cells, contrast=30.0, radius=0.25, seed=3)
+    out, runs = [], []
+    for rep in ((1, 1, 1), repeat):
+        s = np.tile(state.reshape(8, *cells[::-1]), (1, *rep[::-1]))
+        n = tuple(c * r for c, r in zip(cells, rep))
+        with Grid(n, length, gamma, mu0) as g:
+            g.upload(s.reshape(8, -1))
+            g.set_substepping(0, 2)
+            runs.append(g.run("hlld-athena", 0.3, 0.0, 1e9, max_steps=2))
+            out.append(g.download().reshape(8, *n[::-1]))
+    assert runs[0] == runs[1]
+    np.testing.assert_array_equal(out[1], np.tile(out[0], (1, *repeat[::-1])))
