@@ -17,7 +17,10 @@ One step = dt_kernel (1 thread: lagged CFL step from the previous pass) ->
 flux_pass_kernel (one thread per face, all faces of one dimension in a
 z-slab of blocks) -> update_cell_kernel or update_column_kernel (one thread
 per cell, or column tiles marching in z: constrained-transport face update,
-conserved update, constant-pressure energy refits).  In mixed precision the flux array holds FP32 values.
+conserved update, constant-pressure energy refits).  In mixed precision the
+flux array holds FP32 values.  HLLD accumulates in marches instead
+(launch_accumulate), and grids of up to 2^20 cells step in two launches
+(flat_step).
 */
 #include <hip/hip_runtime.h>
 
