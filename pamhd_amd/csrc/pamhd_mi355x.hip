@@ -3802,7 +3802,12 @@ struct pamhd_handle {
 		   is small (flat_step) and no launch variant was asked for */
 		int flat = -1;
 	} tune;
-	bool lag_ok = false;   /* dt holds the last flux pass's reduced speeds and the other status is cleared */
+	/* dt holds the last flux pass's reduced speeds and the other status is
+	   cleared; never true once a step other than a flat one was captured
+	   (marches_captured): a replay of it moves the speeds on in the status
+	   alone, and the host does not see when */
+	bool lag_ok = false;
+	bool marches_captured = false;
 	double* emf = nullptr;     /* 6 x n field components of the fused step, allocated on first use */
 	/* second stream and events of the slab pipeline, created on first use */
 	hipStream_t aux = nullptr;
@@ -4202,17 +4207,23 @@ bool flat_step(const pamhd_handle* h)
 	return h->tune.flat >= 0 ? h->tune.flat == 1 : h->g.n <= 1ll << 20;
 }
 
+bool stream_captures(hipStream_t st)
+{
+	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+	(void)hipStreamIsCapturing(st, &cap);
+	return cap != hipStreamCaptureStatusNone;
+}
+
 template <class T>
 int launch_flat(pamhd_handle* h, int solver, hipStream_t st, double max_dt, double cfl, int refits,
 	int fixed_dt, bool report, StepStatus* prev, StepStatus* next, StepStatus* clear)
 {
-	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-	(void)hipStreamIsCapturing(st, &cap);
-	const bool captured = cap != hipStreamCaptureStatusNone;
+	const bool captured = stream_captures(st);
 	DtRec* rec = reinterpret_cast<DtRec*>(h->dt);
 	/* a captured step may run after any other one: it reduces the speeds
 	   itself, and so does the step after the capture */
 	if (!h->lag_ok || captured) lag_kernel<<<1, NSLOT, 0, st>>>(prev, next, rec);
+	h->lag_ok = false;
 	const FlatGrid fg{flat_div((unsigned)h->g.nx), flat_div((unsigned)h->g.ny)};
 	const unsigned nb = (unsigned)((h->g.n + FLAT - 1) / FLAT);
 	const double* s = h->state[h->cur];
@@ -4228,8 +4239,8 @@ int launch_flat(pamhd_handle* h, int solver, hipStream_t st, double max_dt, doub
 	flat_update_kernel<<<nb + 1, FLAT, 0, st>>>(h->g, fg, s, h->state[1 - h->cur], h->flux, refits,
 		std::is_same_v<T, double> ? h->pe_out : nullptr, next, clear, rec, h->host_dt,
 		report ? h->host_status : nullptr);
-	h->lag_ok = !captured;
 	HIP_TRY(h, hipGetLastError());
+	h->lag_ok = !captured && !h->marches_captured;
 	return PAMHD_OK;
 }
 
@@ -4794,6 +4805,7 @@ int do_step(pamhd_handle* h, int solver, double max_dt, double cfl, int refits,
 		if (e) return e;
 	} else {
 		h->lag_ok = false;
+		if (stream_captures(st)) h->marches_captured = true;
 		{
 			TimedLaunch t(h, st, K_DT);
 			dt_kernel<<<1, NSLOT, 0, st>>>(prev, next, h->dt, cfl, max_dt, h->g.dx, h->g.dy, h->g.dz, fixed_dt);

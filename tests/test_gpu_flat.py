@@ -153,6 +153,37 @@ def test_flat_step_replays_in_a_graph(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["passes", "accumulate"])
+def test_replayed_marches_between_flat_steps(gpu, mode):
+    """two captured steps of another structure, replayed with eager flat
+    steps in between: the flat steps' lagged length follows the replay"""
+    import torch
+    from pamhd_amd import solver as S
+    cells = (33, 7, 5)
+    state, length, gamma, mu0 = _state(cells)
+    with S.Grid(cells, length, gamma, mu0) as a, S.Grid(cells, length, gamma, mu0) as b:
+        for g in (a, b):
+            g.set_fused_step(mode)
+            g.upload(state)
+            g.timestep("hlld-athena", 0.0, 0.3)
+            g.step("hlld-athena", 1e300, 0.3)
+        graph = torch.cuda.CUDAGraph()
+        side = torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=side):
+            for _ in range(2):
+                a.step("hlld-athena", 1e300, 0.3, sync=False, stream=side.cuda_stream)
+        a.set_launch(128)
+        for rep in range(4):
+            for _ in range(2):
+                assert a.step("hlld-athena", 1e300, 0.3) == b.step("hlld-athena", 1e300, 0.3)
+            graph.replay()
+            torch.cuda.synchronize()
+            for _ in range(2):
+                b.step("hlld-athena", 1e300, 0.3)
+            np.testing.assert_array_equal(a.download(), b.download())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["launches", "graph", "persistent"])
 def test_box_cells_by_flat_index(gpu, mode):
     """solar-wind boxes with their default blocks of 256 consecutive cells,
