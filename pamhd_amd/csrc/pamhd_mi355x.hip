@@ -3822,6 +3822,11 @@ struct pamhd_handle {
 	double* adj = nullptr;    /* adjoint scratch, allocated on first use */
 	PoissonMG* mg = nullptr;  /* multigrid hierarchy, allocated on first cleaning */
 	SubstepDev* sub = nullptr; /* per-cell substepping, allocated when enabled */
+	/* grids with boundaries: the cells' types on the host, and whether the
+	   boundaries write the density, velocity or pressure of a normal cell
+	   (a value set on it, or a copy cell of type 1), which copies may read */
+	std::vector<signed char> cell_type;
+	bool normal_copied = false, normal_written = false;
 	int mg_fused = 0;   /* per-colour passes (faster; see pamhd_set_poisson_smoother) */
 	int adj_reverse = 1;   /* flux Jacobian of the adjoint: 1 reverse accumulation, 0 dual numbers */
 	int flux_step = 0;     /* the last step left its FP64 dt * F in flux (pamhd_get_magnetic_fluxes) */
@@ -4306,11 +4311,13 @@ apply_boundaries on a grid with boundaries (source/mhd/boundaries.hpp:
 1261-1297): value and copy boundaries of number density, velocity and
 pressure (apply_fluid_boundaries, :738-1026), of the face field
 (apply_magnetic_field_boundaries_staggered, :250-640, uniform grids), then
-update_vol_B(0) at constant pressure of every cell of type >= 0.  A stage
-before that writes only boundary cells and reads only its own cell and
-normal cells, which none of them writes, so a thread takes its cell through
-all of them (bnd_apply_kernel).  Neighbours are visited in the order of the
-neighbourhood (offsets -1..1, z slowest).
+update_vol_B(0) at constant pressure of every cell of type >= 0.  Where the
+value and copy cells are boundary cells, a stage before that writes only
+boundary cells and reads only its own cell and normal cells, which none of
+them writes, so a thread takes its cell through all of them
+(bnd_apply_kernel); a caller may also put values on normal cells
+(normal_written), then the copies wait for each stage's values.  Neighbours
+are visited in the order of the neighbourhood (offsets -1..1, z slowest).
 */
 struct BndNb { int id; int fn; int en0, en1, en2; };
 
@@ -4359,29 +4366,37 @@ __device__ __forceinline__ double bnd_pressure(const SubstepDev& d, long long n,
 	return pressure64(U, ph.gm1, ph.half_inv_mu0);
 }
 
-/* STAGE 0 number density, 1 velocity, 2 pressure */
+/* STAGE 0 number density, 1 velocity, 2 pressure: the cell's value; false
+   after an error */
 template <int STAGE>
-__device__ __forceinline__ void bnd_fluid(const GridDev& g, const SubstepDev& d, double proton_mass, int i,
+__device__ __forceinline__ bool bnd_value(const GridDev& g, const SubstepDev& d, double proton_mass, int i,
 	int j, int k)
 {
 	const long long n = g.n;
 	const int c = cidx(g, i, j, k);
-	if (d.bmask[STAGE * n + c]) {
-		if (STAGE == 0) {
-			d.S[c] = proton_mass * d.bval[c];
-		} else if (STAGE == 1) {
-			for (int q = 0; q < 3; q++) d.S[(1 + q) * n + c] = d.bval[(1 + q) * n + c] * d.S[c];
-		} else {
-			if (d.S[c] <= 0) { record_error(d.status, PAMHD_E_DENSITY, 2 * n + c); return; }
-			double v[3];
-			bnd_velocity(d, n, c, v);
-			const double B[3] = {d.S[5 * n + c], d.S[6 * n + c], d.S[7 * n + c]};
-			d.S[4 * n + c] = total_energy64(d.S[c], v, d.bval[4 * n + c], B, g.ph.gm1, g.ph.half_inv_mu0);
-		}
+	if (!d.bmask[STAGE * n + c]) return true;
+	if (STAGE == 0) {
+		d.S[c] = proton_mass * d.bval[c];
+	} else if (STAGE == 1) {
+		for (int q = 0; q < 3; q++) d.S[(1 + q) * n + c] = d.bval[(1 + q) * n + c] * d.S[c];
+	} else {
+		if (d.S[c] <= 0) { record_error(d.status, PAMHD_E_DENSITY, 2 * n + c); return false; }
+		double v[3];
+		bnd_velocity(d, n, c, v);
+		const double B[3] = {d.S[5 * n + c], d.S[6 * n + c], d.S[7 * n + c]};
+		d.S[4 * n + c] = total_energy64(d.S[c], v, d.bval[4 * n + c], B, g.ph.gm1, g.ph.half_inv_mu0);
 	}
+	return true;
+}
+
+/* the same stages' copies: the average over normal face neighbours, else
+   over normal edge neighbours */
+template <int STAGE>
+__device__ __forceinline__ void bnd_copy(const GridDev& g, const SubstepDev& d, int i, int j, int k)
+{
+	const long long n = g.n;
+	const int c = cidx(g, i, j, k);
 	if (d.vt[STAGE * n + c] != 4) return;
-	/* copy: the average over normal face neighbours, else over normal
-	   edge neighbours */
 	double fs[3] = {0, 0, 0}, es[3] = {0, 0, 0};
 	unsigned long long nf = 0, ne = 0;
 	bool bad = false;
@@ -4481,14 +4496,35 @@ __device__ __forceinline__ void bnd_field_copy(const GridDev& g, const SubstepDe
 
 /* the stages of one cell in order: each writes only its own cell (a boundary
    cell; its faces of type 1 with the values they have) and reads that cell
-   and what no stage changes (normal cells, faces of type 1) */
+   and what no stage changes (normal cells, faces of type 1).  Not where a
+   normal cell is written (normal_written) */
 __global__ __launch_bounds__(BX * BY) void bnd_apply_kernel(GridDev g, SubstepDev d, double proton_mass)
 {
 	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
 	if (i >= g.nx || j >= g.ny) return;
-	bnd_fluid<0>(g, d, proton_mass, i, j, k);
-	bnd_fluid<1>(g, d, proton_mass, i, j, k);
-	bnd_fluid<2>(g, d, proton_mass, i, j, k);
+	if (bnd_value<0>(g, d, proton_mass, i, j, k)) bnd_copy<0>(g, d, i, j, k);
+	if (bnd_value<1>(g, d, proton_mass, i, j, k)) bnd_copy<1>(g, d, i, j, k);
+	if (bnd_value<2>(g, d, proton_mass, i, j, k)) bnd_copy<2>(g, d, i, j, k);
+	bnd_field_value(g, d, i, j, k);
+	bnd_field_copy(g, d, i, j, k);
+}
+
+/* one stage's values, or its copies, of every cell (normal_written) */
+template <int STAGE, bool COPY>
+__global__ __launch_bounds__(BX * BY) void bnd_stage_kernel(GridDev g, SubstepDev d, double proton_mass)
+{
+	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
+	if (i >= g.nx || j >= g.ny) return;
+	if constexpr (COPY) bnd_copy<STAGE>(g, d, i, j, k);
+	else (void)bnd_value<STAGE>(g, d, proton_mass, i, j, k);
+}
+
+/* the face field's stages alone: they read faces of type 1, which no stage
+   changes whatever cells have values */
+__global__ __launch_bounds__(BX * BY) void bnd_field_kernel(GridDev g, SubstepDev d)
+{
+	const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y, k = blockIdx.z;
+	if (i >= g.nx || j >= g.ny) return;
 	bnd_field_value(g, d, i, j, k);
 	bnd_field_copy(g, d, i, j, k);
 }
@@ -4660,7 +4696,18 @@ void launch_boundaries(pamhd_handle* h, hipStream_t st)
 {
 	SubstepDev& d = *h->sub;
 	const dim3 grid = cell_grid(h->g), block(BX, BY, 1);
-	bnd_apply_kernel<<<grid, block, 0, st>>>(h->g, d, h->phys.proton_mass);
+	const double mp = h->phys.proton_mass;
+	if (h->normal_written) {
+		bnd_stage_kernel<0, false><<<grid, block, 0, st>>>(h->g, d, mp);
+		bnd_stage_kernel<0, true><<<grid, block, 0, st>>>(h->g, d, mp);
+		bnd_stage_kernel<1, false><<<grid, block, 0, st>>>(h->g, d, mp);
+		bnd_stage_kernel<1, true><<<grid, block, 0, st>>>(h->g, d, mp);
+		bnd_stage_kernel<2, false><<<grid, block, 0, st>>>(h->g, d, mp);
+		bnd_stage_kernel<2, true><<<grid, block, 0, st>>>(h->g, d, mp);
+		bnd_field_kernel<<<grid, block, 0, st>>>(h->g, d);
+	} else {
+		bnd_apply_kernel<<<grid, block, 0, st>>>(h->g, d, mp);
+	}
 	bnd_refit_kernel<<<grid, block, 0, st>>>(h->g, d);
 	ss_sync_kernel<<<cell_grid_and_plane(h->g), block, 0, st>>>(h->g, d, d.host_status);
 	ss_end(h, false, st);
@@ -4964,6 +5011,10 @@ int pamhd_create_bounded(const pamhd_grid_desc* grid, const pamhd_physics* physi
 	for (int q = 0; q < 3; q++) d.per[q] = grid->periodic[q] ? 1 : 0;
 	d.smax = 0;
 	d.opt = nullptr;
+	h->cell_type.assign(cell_type, cell_type + n);
+	for (long long q = 0; q < 3 * n; q++)
+		if (var_type[q] == 4 && cell_type[q % n] >= 1) h->normal_copied = true;
+	h->normal_written = h->normal_copied;
 	*out = h;
 	return PAMHD_OK;
 }
@@ -4978,6 +5029,10 @@ int pamhd_set_boundary_values(pamhd_handle* h, const unsigned char* mask, const 
 	if (!h->sub || !h->sub->bounded) return fail(h, PAMHD_E_ARG, "not a grid with boundaries");
 	SubstepDev& d = *h->sub;
 	const size_t n = (size_t)h->g.n;
+	int normal = 0;
+	for (size_t c = 0; c < n; c++)
+		normal |= (h->cell_type[c] >= 1) & ((mask[c] | mask[n + c] | mask[2 * n + c]) != 0);
+	h->normal_written = h->normal_copied || normal;
 	HIP_TRY(h, hipMemcpy(d.bmask, mask, 4 * n, hipMemcpyHostToDevice));
 	HIP_TRY(h, hipMemcpy(d.bval, number_density, sizeof(double) * n, hipMemcpyHostToDevice));
 	HIP_TRY(h, hipMemcpy(d.bval + n, velocity, sizeof(double) * 3 * n, hipMemcpyHostToDevice));
