@@ -2523,7 +2523,7 @@ struct SubstepDev {
 	unsigned long long* scal = nullptr;
 	double* sub_dt = nullptr;
 	StepStatus* status = nullptr;
-	unsigned long long* host = nullptr;   /* pinned: [0] largest period, [1] substep length (bits), [2] largest level */
+	unsigned long long* host = nullptr;   /* pinned: [0] largest period (0: not known yet), [1] substep length (bits), [2] largest level */
 	StepStatus* host_status = nullptr;
 	int smax = 0;   /* uniform substep-max, or the largest per-cell one */
 	int last_max = 1;
@@ -2915,9 +2915,20 @@ blocks' minima (22 us of it those, waited for at the end), 19 us with LDS for
 both, 9.8 us without the passes that cannot matter when all periods are 1.
 A step of that tube: 9 launches, 4 copies and a host wait less; 175 us
 before, 76 us with this and the merged passes.
+
+A restriction pass and the minima around the cells cost the block some 10 us
+per cell of a thread, the grid's kernels 4 us whatever the cells.  So with
+more than a cell a thread (SS_PREP_LEVELS) and levels above 0 the block
+stops at the levels and leaves host[0] at 0, and the host goes on with the
+grid's kernels.  us per HLL step with the largest period 4, the grid's
+kernels alone / all in the block / the block up to the levels: 2000 x 1 x 1
+232 / 218 / 206, 16^3 256 / 293 / 228, 128 x 128 x 1 246 / 626 / 236 (1000 x 1
+x 1 in the block 200, the grid's kernels 239); with all periods 1, the
+grid's kernels / the block: 16^3 114 / 65, 128 x 128 x 1 114 / 89.
 */
 constexpr int SS_PREP = 1024;
 constexpr int SS_PREP_CELLS = 16 * SS_PREP;
+constexpr int SS_PREP_LEVELS = SS_PREP;   /* cells that the block restricts itself, at most */
 constexpr int SS_PREP_BLOCKS = 1024;   /* blocks of the cell grid, at most */
 
 __global__ __launch_bounds__(SS_PREP) void ss_prep_kernel(GridDev g, FlatGrid fg, SubstepDev d, double cfl,
@@ -3049,6 +3060,21 @@ __global__ __launch_bounds__(SS_PREP) void ss_prep_kernel(GridDev g, FlatGrid fg
 	}
 	/* (block_max's barriers end the pass) */
 	const int passes = block_max(most);
+	const double sub_dt = all_zero ? max_dt : r;
+	if (tid == 0) {
+		*d.sub_dt = sub_dt;
+		host[1] = (unsigned long long)__double_as_longlong(sub_dt);
+		host[2] = (unsigned long long)passes;
+		/* written by atomics and stores of other waves */
+		host_status->err = __hip_atomic_load(&d.status->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		host_status->err_face = __hip_atomic_load(&d.status->err_face, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
+	if (passes > 0 && n > SS_PREP_LEVELS) {
+		for (int s = tid; s < SS_SLOTS; s += SS_PREP) d.scal[1 * SS_SLOTS + s] = 0;
+		for (int c = tid; c < n; c += SS_PREP) d.e[0][c] = lev_s[0][c] == P_NONE ? 0 : (int)lev_s[0][c];
+		if (tid == 0) host[0] = 0;
+		return;
+	}
 	int cur = 0;
 	for (int q = 0; q < passes; q++) {
 		for (int c = tid; c < n; c += SS_PREP) {
@@ -3097,15 +3123,7 @@ __global__ __launch_bounds__(SS_PREP) void ss_prep_kernel(GridDev g, FlatGrid fg
 		__syncthreads();
 		for (int b = tid; b < 4 * d.nblk; b += SS_PREP) d.blk[b] = blk_s[b];
 	}
-	if (tid == 0) {
-		const double sub_dt = all_zero ? max_dt : r;
-		*d.sub_dt = sub_dt;
-		host[0] = (unsigned long long)largest;
-		host[1] = (unsigned long long)__double_as_longlong(sub_dt);
-		/* written by atomics and stores of other waves */
-		host_status->err = __hip_atomic_load(&d.status->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		host_status->err_face = __hip_atomic_load(&d.status->err_face, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-	}
+	if (tid == 0) host[0] = (unsigned long long)largest;
 }
 
 /*
@@ -4721,11 +4739,10 @@ int substep_step(pamhd_handle* h, int solver, double max_dt, double cfl, int ref
 	SubstepDev& d = *h->sub;
 	const dim3 grid = cell_grid(h->g), block(BX, BY, 1);
 	double* P = h->flux;   /* the substep's field components per face, 6 x n (of 24 x n) */
-	if (h->g.n <= SS_PREP_CELLS && d.nblk <= SS_PREP_BLOCKS) {
+	const bool prep = h->g.n <= SS_PREP_CELLS && d.nblk <= SS_PREP_BLOCKS;
+	if (prep) {
 		ss_prep_kernel<<<1, SS_PREP, 0, st>>>(h->g, FlatGrid{flat_div((unsigned)h->g.nx), flat_div((unsigned)h->g.ny)}, d, cfl, max_dt, d.host, d.host_status);
 		HIP_TRY(h, hipGetLastError());
-		HIP_TRY(h, hipStreamSynchronize(st));
-		if (d.host_status->err) return report_status(h, *d.host_status);
 	} else {
 		ss_clear_kernel<<<1, SS_FOLD, 0, st>>>(d);
 		ss_ts_kernel<<<grid, block, 0, st>>>(h->g, d, cfl);
@@ -4736,8 +4753,10 @@ int substep_step(pamhd_handle* h, int solver, double max_dt, double cfl, int ref
 		HIP_TRY(h, hipGetLastError());
 		HIP_TRY(h, hipMemcpyAsync(d.host + 2, d.scal + 3 * SS_SLOTS, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
 		HIP_TRY(h, hipMemcpyAsync(d.host_status, d.status, sizeof(StepStatus), hipMemcpyDeviceToHost, st));
-		HIP_TRY(h, hipStreamSynchronize(st));
-		if (d.host_status->err) return report_status(h, *d.host_status);
+	}
+	HIP_TRY(h, hipStreamSynchronize(st));
+	if (d.host_status->err) return report_status(h, *d.host_status);
+	if (!prep || d.host[0] == 0) {
 		/* Jacobi passes of the restriction: a cell's restricted level is the
 		   smallest over cells m of level(m) + distance, reached within as many
 		   passes as the largest level */

@@ -208,10 +208,12 @@ def test_box_cells_by_flat_index(gpu, mode):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("cells", [(2, 3, 900), (2, 3, 1200), (65, 5, 4), (1, 1, 65535), (32, 32, 17)])
+@pytest.mark.parametrize("cells", [(2, 3, 900), (2, 3, 1200), (65, 5, 4), (1, 1, 65535), (32, 32, 17),
+                                   (32, 32, 1), (41, 25, 1)])
 def test_substep_preparation_paths(gpu, cells):
     """substepped steps of grids around the limits of the one-block
-    preparation (16384 cells, 1024 blocks of 64 x 4 cells) and with the most
+    preparation (16384 cells, 1024 blocks of 64 x 4 cells; 1024 cells for its
+    restriction of the levels) and with the most
     planes a launch has (no plane of blocks past them), against the oracle"""
     from pamhd_amd import configs
     from pamhd_amd import solver as S
