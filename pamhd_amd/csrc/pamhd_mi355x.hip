@@ -4655,14 +4655,18 @@ dim3 ss_walk_grid(const SubstepDev& d)
 /* the flux passes of substep `sub`; at a substep where every face is due
    (full) they cover the whole cell grid, and no edge field needs zeroing.
    Up to 2^20 cells the three directions share a launch (per face: marches
-   leave the GPU idle there, as in flat_step) */
+   leave the GPU idle there, as in flat_step).  Roe's shared kernel needs
+   more than 256 registers and runs one wave on a SIMD, two with a kernel
+   per direction, so it shares a launch only while the launches themselves
+   count (us per step, shared -> a launch each: 16^3 69 -> 88, 32^3 127 -> 131,
+   48^3 186 -> 181, 64^3 251 -> 220, 100^3 850 -> 643) */
 template <int SOLVER>
 void ss_launch_flux(pamhd_handle* h, double* P, int sub, bool full, hipStream_t st)
 {
 	const SubstepDev& d = *h->sub;
 	const dim3 block(BX, BY, 1);
 	if (full) {
-		if (h->g.n <= 1ll << 20) {
+		if (h->g.n <= (SOLVER == ROE_ATHENA ? 1ll << 16 : 1ll << 20)) {
 			ss_flux3_kernel<SOLVER, false><<<dim3((unsigned)d.nblk, 3, 1), block, 0, st>>>(h->g, d, h->bg, P, sub);
 			return;
 		}

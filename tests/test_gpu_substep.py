@@ -256,3 +256,21 @@ def test_full_passes_of_large_grids(gpu, repeat):
             out.append(g.download().reshape(8, *n[::-1]))
     assert runs[0] == runs[1]
     np.testing.assert_array_equal(out[1], np.tile(out[0], (1, *repeat[::-1])))
+
+
+@pytest.mark.parametrize("cells", [(64, 32, 32), (64, 32, 33)])
+def test_roe_full_passes_bit_exact(gpu, cells):
+    """Roe's passes over every face: one launch up to 2^16 cells, one per
+    direction above"""
+    from pamhd_amd.solver import Grid
+    state, length, gamma, mu0 = configs.hot_blob(cells, contrast=30.0, radius=0.25, seed=3)
+    ref = state.copy()
+    st, steps, t, largest = O.run_periodic_substep(O.make_grid(cells, length, gamma, mu0), O.ROE, 0.3, 0, 2,
+                                                   0.0, 1e9, ref, max_steps=3)
+    assert st == 0 and largest > 1
+    with Grid(cells, length, gamma, mu0) as g:
+        g.upload(state)
+        g.set_substepping(0, 2)
+        print("cells", cells, flush=True)
+        assert g.run("roe-athena", 0.3, 0.0, 1e9, max_steps=3) == (steps, t)
+        np.testing.assert_array_equal(g.download(), ref)
