@@ -202,7 +202,8 @@ __device__ __forceinline__ double relax_at(const LevelArgs& L, const double* phi
 {
 	if (L.diag.b == 0) return phi[x[0]];
 	double p[7];
-	for (int q = 1; q < 7; q++) p[q] = phi[x[q]];
+	for (int q = 1; q < 5; q++) p[q] = phi[x[q]];
+	if (L.n2 > 1) for (int q = 5; q < 7; q++) p[q] = phi[x[q]];
 	return evaluated(L, [&](auto& quot) {
 		double s = 0;
 		if (L.n0 > 1) s += quot(p[1] + p[2], L.hh0);
@@ -237,7 +238,8 @@ __device__ __forceinline__ double residual_at(const LevelArgs& L, const double* 
 	int x[7];
 	nb7(L, i, j, k, x);
 	double p[7];
-	for (int q = 0; q < 7; q++) p[q] = phi[x[q]];
+	for (int q = 0; q < 5; q++) p[q] = phi[x[q]];
+	if (L.n2 > 1) for (int q = 5; q < 7; q++) p[q] = phi[x[q]];
 	const double fc = f[x[0]];
 	return evaluated(L, [&](auto& quot) { return residual_of(L, p, fc, quot); });
 }
@@ -979,7 +981,9 @@ neighbours are consecutive over the threads in each colour's half, where a
 thread a cell makes every load of a wave two half-used pieces; planes beyond
 the grid are read at its last plane and masked, so that no branch keeps the
 loads of one plane behind those of another.  256^3 cells: 59 us, 95 us with
-a thread a cell; the two arrays take 53 us at a copy's rate.
+a thread a cell; the two arrays take 53 us at a copy's rate.  Grids that
+leave most of a block's planes empty keep a thread a cell
+(norm_planes_filled).
 */
 __global__ __launch_bounds__(PBX * PBY / 2) void norm_packed_kernel(Tiles T, LevelArgs L,
 	const double* __restrict__ phi, const double* __restrict__ f, double* __restrict__ part)
@@ -1340,6 +1344,14 @@ void mg_vcycle(PoissonMG& mg, hipStream_t st, int l)
 	mg_smooth(mg, st, l, 2);
 }
 
+/* whether norm_packed_kernel, which computes NORM_KZ planes whatever the grid
+   has, does less than norm_partial_kernel, which takes about 1.6 times as
+   long for a full plane (1000 x 1000 x 1 cells: 29.5 us, a thread a cell 15.9) */
+bool norm_planes_filled(int n2)
+{
+	return (n2 + NORM_KZ - 1) / NORM_KZ * NORM_KZ * 5 <= 8 * n2;
+}
+
 /* ||r - mean(r)||_2 of the finest level's residual r = f - L phi, or of f
    alone (with_lap 0) */
 static hipError_t centred_norm(PoissonMG& mg, hipStream_t st, int with_lap, double* out)
@@ -1347,7 +1359,7 @@ static hipError_t centred_norm(PoissonMG& mg, hipStream_t st, int with_lap, doub
 	const MgLevel& F = mg.lv[0];
 	Tiles T = tiles_of(F.n[0], F.n[1], (F.n[2] + NORM_KZ - 1) / NORM_KZ);
 	const int nb = blocks_of(T);
-	if (with_lap && F.packed) {
+	if (with_lap && F.packed && norm_planes_filled(F.n[2])) {
 		norm_packed_kernel<<<nb, dim3(PBX / 2, PBY, 1), 0, st>>>(T, args_of(F), F.phi, F.f, mg.norm_part);
 	} else {
 		norm_partial_kernel<<<nb, dim3(PBX, PBY, 1), 0, st>>>(T, args_of(F), F.phi, F.f, with_lap,

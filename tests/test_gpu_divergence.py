@@ -117,6 +117,8 @@ def test_clean_divergence_reports_unconverged(gpu):
 @pytest.mark.parametrize("cells,field,spacing", [
     ((64, 64, 64), 1.0, 1.0), ((66, 6, 10), 1.0, 1.0), ((130, 36, 18), 1.0, 1.0),
     ((32, 8, 8), 1.0, 1.0), ((8, 8, 4), 1.0, 1.0), ((16, 12, 9), 1.0, 1.0),
+    ((66, 6, 1), 1.0, 1.0), ((1, 66, 6), 1.0, 1.0), ((40, 20, 2), 1.0, 1.0), ((64, 20, 4), 1.0, 1.0),
+    ((40, 20, 6), 1.0, 1.0),
     ((40, 20, 12), 1e-148, 1.0), ((40, 20, 12), 1e-150, 1.0), ((40, 20, 12), 1e100, 1.0),
     ((40, 20, 12), 1.0, 1e40)])
 def test_clean_divergence_tiles_and_ranges(gpu, cells, field, spacing):
