@@ -1876,7 +1876,7 @@ path, each finishing its direction's part of update_mhd_state's conserved
 update (source/mhd/solve.hpp:1503-1614) instead of storing face fluxes:
 
   acc_x_kernel      x-faces, a wave per 64 cells of a plane walking km planes
-                    along z (the left part of lane l is lane l - 1's, the
+                    along z, or y on flat grids (the left part of lane l is lane l - 1's, the
                     face of lane l + 1 comes one lane down; the rows'
                     left-edge parts and right-edge face fluxes are computed
                     for all km planes before the march); writes
@@ -1986,8 +1986,9 @@ __host__ __device__ __forceinline__ int acc_segments(int nx)
 
 /*
 x-faces.  A wave takes 64 consecutive cells of the plane's flat index
-i + nx j and marches km planes along z, so rows that are no multiple of 64
-cells leave no lane idle (nx = 200: 22 % of the lanes of 64-cell row tiles).
+i + nx j and marches km planes along z (grids of few z planes: of i + nx k
+along y, march_along_y), so rows that are no multiple of 64 cells leave no
+lane idle (nx = 200: 22 % of the lanes of 64-cell row tiles).
 Where a row starts inside the wave the left part is not the lane below's,
 and where one ends the right face is not the lane above's: those, and the
 wave's own first and last, are computed for all km planes before the march,
@@ -1995,8 +1996,8 @@ one edge and plane per lane (acc_segments(nx) * km <= ACC_EDGE).  Mixed
 200 x 180 x 152 step, row tiles -> flat index (both marches): x 365 -> 304,
 y 391 -> 267, z 301 -> 242 us.
 */
-template <class T, int MINB>
-__global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv div_nx, StateArrays S,
+template <class T, bool ALONG_Y>
+__global__ __launch_bounds__(BX * BY, 1) void acc_x_kernel(GridDev g, FlatDiv div_nx, StateArrays S,
 	double* __restrict__ out, double* __restrict__ emf, const double* __restrict__ dtp,
 	StepStatus* st, unsigned gx, int km, int remap)
 {
@@ -2007,17 +2008,18 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 	const int chunk = (int)(lb / gx);
 	const int lane = threadIdx.x;
 	const int tid = lane + BX * threadIdx.y;
-	const int plane = g.nx * g.ny;
+	const int nt = ALONG_Y ? g.nz : g.ny, na = ALONG_Y ? g.ny : g.nz;
+	const int plane = g.nx * nt;
 	/* the wave's first cell of the plane, its row and column */
 	const int l0 = __builtin_amdgcn_readfirstlane((int)(bx * BY + threadIdx.y) * BX);
-	const int j0 = (int)div_nx((unsigned)l0), i0 = l0 - j0 * g.nx;
+	const int t0 = (int)div_nx((unsigned)l0), i0 = l0 - t0 * g.nx;
 	const bool own = l0 + lane < plane;
 	const int l = min(l0 + lane, plane - 1);   /* lanes past the plane repeat its last cell */
-	const int j = (int)div_nx((unsigned)l), i = l - j * g.nx;
-	const int seg = j - j0;
+	const int t = (int)div_nx((unsigned)l), i = l - t * g.nx;
+	const int seg = t - t0;
 	const bool row_start = i == 0, row_end = i + 1 == g.nx;
 	const int a0 = chunk * km;
-	const int a1 = min(a0 + km, g.nz);
+	const int a1 = min(a0 + km, na);
 	const size_t n = g.n;
 	double sp = 0;
 	unsigned zero = 0;
@@ -2031,19 +2033,19 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 		const double dt = *dtp;
 		const double il = 1 / g.dx;
 		const int planes = a1 - a0;
-		const int segs = min((i0 + BX - 1) / g.nx + 1, g.ny - j0);
+		const int segs = min((i0 + BX - 1) / g.nx + 1, nt - t0);
 		if (lane < segs * planes) {
 			const int sg = lane / planes, a = a0 + lane % planes;
-			const int row = j0 + sg;
+			const int row = ALONG_Y ? a : t0 + sg, pl = ALONG_Y ? t0 + sg : a;
 			const int first = sg == 0 ? i0 : 0;
 			const int last = min(i0 + BX - 1 - sg * g.nx, g.nx - 1);
 			double U[8];
-			load_face_state_d<0>(S, g, wrap_dec(first, g.nx), row, a, U);
+			load_face_state_d<0>(S, g, wrap_dec(first, g.nx), row, pl, U);
 			apart_make<T>(U, g.ph, edge_l[threadIdx.y][lane]);
 			P pa, pb;
-			load_face_state_d<0>(S, g, last, row, a, U);
+			load_face_state_d<0>(S, g, last, row, pl, U);
 			apart_make<T>(U, g.ph, pa);
-			load_face_state_d<0>(S, g, wrap_inc(last, g.nx), row, a, U);
+			load_face_state_d<0>(S, g, wrap_inc(last, g.nx), row, pl, U);
 			apart_make<T>(U, g.ph, pb);
 			double s_unused;
 			apart_face<T, 0>(pa, pb, g.ph, dt, edge_r[threadIdx.y][lane].f, s_unused);
@@ -2052,6 +2054,7 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 		for (int a = a0; a < a1; a++) {
 			double s_face;
 			int e;
+			const int j = ALONG_Y ? a : t, k = ALONG_Y ? t : a;
 			const int at = a - a0, mine = min(seg, segs - 1) * planes + at;
 			if constexpr (std::is_same_v<T, double>) {
 				/* FP64: the face of the lane above comes down with a DPP
@@ -2060,7 +2063,7 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 				double lo[8], hi[8];
 				{
 					double U[8];
-					load_face_state_d<0>(S, g, i, j, a, U);
+					load_face_state_d<0>(S, g, i, j, k, U);
 					P R;
 					apart_make<T>(U, g.ph, R);
 					P L = apart_up(R, edge_l[threadIdx.y][at]);
@@ -2075,13 +2078,13 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 					for (int q = 0; q < 8; q++) hi[q] = edge_r[threadIdx.y][mine].f[q];
 				}
 				if (own) {
-					const int c = l + plane * a;
+					const int c = i + g.nx * (j + g.ny * k);
 					double U[8];
 					if (e) record_error(st, e, (long long)c);
 					sp = smax(sp, s_face);
 					zero += s_face <= 0 ? 1u : 0u;
 					store_emf<0>(emf, n, c, lo);
-					load_face_state_d<0>(S, g, i, j, a, U);
+					load_face_state_d<0>(S, g, i, j, k, U);
 					add_terms<double>(U, lo, hi, g.dx, il);
 #pragma unroll
 					for (int q = 0; q < 8; q++) out[q * n + c] = U[q];
@@ -2090,7 +2093,7 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 			}
 			{
 				double U[8];
-				load_face_state_d<0>(S, g, i, j, a, U);
+				load_face_state_d<0>(S, g, i, j, k, U);
 				P R;
 				apart_make<T>(U, g.ph, R);
 				P L = apart_up(R, edge_l[threadIdx.y][at]);
@@ -2107,7 +2110,7 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 			__asm__ volatile("" ::: "memory");
 			__builtin_amdgcn_wave_barrier();
 			if (own) {
-				const int c = l + plane * a;
+				const int c = i + g.nx * (j + g.ny * k);
 				double lo[8], hi[8], U[8];
 				const bool last = row_end || lane == BX - 1;
 				const int up = last ? tid : tid + 1;
@@ -2120,7 +2123,7 @@ __global__ __launch_bounds__(BX * BY, MINB) void acc_x_kernel(GridDev g, FlatDiv
 				sp = smax(sp, s_face);
 				zero += s_face <= 0 ? 1u : 0u;
 				store_emf<0>(emf, n, c, lo);
-				load_face_state_d<0>(S, g, i, j, a, U);
+				load_face_state_d<0>(S, g, i, j, k, U);
 				add_terms<double>(U, lo, hi, g.dx, il);
 #pragma unroll
 				for (int q = 0; q < 8; q++) out[q * n + c] = U[q];
@@ -4179,6 +4182,20 @@ int march_cells(unsigned blocks, int nd, int resident, int most)
 	return best;
 }
 
+/*
+Whether the x march walks y instead of z: its row edges are computed before
+the march, a part and a half of a wave's work for a plane, so z needs planes
+enough, and a plane of x and z cells to fill the waves.  us per HLLD step
+along z -> along y, FP64 (mixed): 2048 x 2048 x 1 1254 -> 1050 (978 -> 823),
+2048 x 1024 x 2 1005 -> 912 (855 -> 781), 1024 x 1024 x 4 908 -> 877 (782 ->
+756), 700 x 500 x 8 601 -> 591 (527 -> 522), 1000 x 350 x 12 890 -> 886 (782
+-> 792), 16 x 131072 x 1 1483 -> 2299.
+*/
+bool march_along_y(const GridDev& g)
+{
+	return g.nz <= 8 && g.ny > g.nz && g.nx * g.nz >= 1024;
+}
+
 /* the accumulating step: x, y and z marches into state[1 - cur], then the
    face-field update and refits */
 template <class T>
@@ -4197,13 +4214,16 @@ int launch_accumulate(pamhd_handle* h, hipStream_t st, StepStatus* next, int ref
 	const unsigned gxy = blocks((long long)h->g.nx * h->g.ny), gxz = blocks((long long)h->g.nx * h->g.nz);
 	/* x: 2 waves per SIMD resident, at most ACC_EDGE row edges per wave */
 	const int edges = std::max(1, ACC_EDGE / acc_segments(h->g.nx));
-	const int kx = h->tune.acc_km > 0 ? std::min(h->tune.acc_km, edges) : march_cells(gxy, h->g.nz, 2, std::min(edges, ACC_KMAX));
+	const bool ay = march_along_y(h->g);
+	const int nx_march = ay ? h->g.ny : h->g.nz;
+	const unsigned gx = ay ? gxz : gxy;
+	const int kx = h->tune.acc_km > 0 ? std::min(h->tune.acc_km, edges) : march_cells(gx, nx_march, 2, std::min(edges, ACC_KMAX));
 	const int ky = h->tune.acc_km > 0 ? h->tune.acc_km : march_cells(gxz, h->g.ny, 3, ACC_KMAX);
 	const int kz = h->tune.acc_km > 0 ? h->tune.acc_km : march_cells(gxy, h->g.nz, 3, ACC_KMAX);
 	{
 		TimedLaunch t(h, st, K_FLUX);
-		acc_x_kernel<T, 1><<<gxy * ((h->g.nz + kx - 1) / kx), block, 0, st>>>(h->g, dx, S, out, h->emf, h->dt,
-			next, gxy, kx, r);
+		auto x_march = ay ? acc_x_kernel<T, true> : acc_x_kernel<T, false>;
+		x_march<<<gx * ((nx_march + kx - 1) / kx), block, 0, st>>>(h->g, dx, S, out, h->emf, h->dt, next, gx, kx, r);
 		acc_march_kernel<T, 1, 3><<<gxz * ((h->g.ny + ky - 1) / ky), block, 0, st>>>(h->g, dx, S, out, h->emf,
 			h->dt, next, gxz, ky, r, refits);
 		acc_march_kernel<T, 2, 3><<<gxy * ((h->g.nz + kz - 1) / kz), block, 0, st>>>(h->g, dx, S, out, h->emf,

@@ -83,6 +83,24 @@ def test_fused_mixed_matches_two_pass_mixed(gpu, cells):
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("cells", [(1024, 40, 1), (1030, 9, 1), (345, 70, 3), (130, 9, 8)])
+def test_x_march_along_y(gpu, cells):
+    """flat grids of at least 1024 cells of x and z, whose x pass marches
+    along y: FP64 against the oracle, mixed against the flux passes"""
+    print("cells", cells, flush=True)
+    state, length, gamma, mu0 = _state(cells, 5)
+    ref = state.copy()
+    st, steps_o, t_o = O.run_periodic(O.make_grid(cells, length, gamma, mu0), O.HLLD, 0.3, 0.0, 1e9, ref, max_steps=3)
+    assert st == 0
+    out, n, t, _, _ = _run(cells, 3, "accumulate")
+    assert (n, t) == (steps_o, t_o)
+    np.testing.assert_array_equal(out, ref)
+    a = _run(cells, 3, "accumulate", precision="mixed")
+    b = _run(cells, 3, "passes", precision="mixed")
+    assert a[1:3] == b[1:3]
+    np.testing.assert_array_equal(a[0], b[0])
+
+
 def test_fused_reports_the_failing_face(gpu):
     """A cell of negative thermal pressure: every step structure fails with
     the pressure error on a face of that cell (which of the cell's faces is
