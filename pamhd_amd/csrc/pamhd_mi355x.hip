@@ -1367,7 +1367,10 @@ __global__ __launch_bounds__(NSLOT) void lag_kernel(StepStatus* cur, StepStatus*
 }
 
 /* cells / FLAT blocks update the cells, the last block ends the pass; host
-   (pinned, may be null) receives the step length and the error */
+   (pinned, may be null) receives the step length and the error.  The
+   blocks take the cells in the XCD-aware order, so that the rows and planes
+   around a block's are read through the same L2: HLL mixed, 512 x 512 x 2
+   103 -> 89 us a step, 512 x 512 x 4 200 -> 186 */
 __global__ __launch_bounds__(FLAT) void flat_update_kernel(GridDev g, FlatGrid fg,
 	const double* __restrict__ s, double* __restrict__ out, const double* __restrict__ P, int refits,
 	double* __restrict__ pe, StepStatus* cur, StepStatus* other, DtRec* rec, double* host_dt,
@@ -1390,7 +1393,7 @@ __global__ __launch_bounds__(FLAT) void flat_update_kernel(GridDev g, FlatGrid f
 		}
 		return;
 	}
-	const int c = (int)blockIdx.x * FLAT + threadIdx.x;
+	const int c = (int)logical_block(blockIdx.x, gridDim.x - 1) * FLAT + threadIdx.x;
 	if (c >= (int)g.n) return;
 	int i, j, k;
 	fg.cell(g, c, i, j, k);
@@ -4241,13 +4244,24 @@ cells they leave SIMDs without a wave.  us per step, marches -> flat:
   HLLD  48^3 76 -> 36, 64^3 95 -> 65, 96^3 204 -> 204, 112^3 295 -> 330
   HLL   20x20 26 -> 12, 64^3 139 -> 54, 96^3 238 -> 170, 128^3 376 -> 418
   Roe   20x20 33 -> 15, 64^3 101 -> 82, 96^3 328 -> 267, 128^3 605 -> 621
-so all cross over at about 100^3 cells.  Kernel timing keeps the launches it
-accounts for.
+so all cross over at about 100^3 cells, in mixed precision too (512 x 512 x 2
+HLL 90 -> 84, 256 x 256 x 16 196 -> 186, 1024 x 1024 x 1 180 -> 181).  With a
+background field (Rusanov and HLL) both sides fetch it per face, and from
+2^19 cells on the column update gains if its 128 x 2 tiles are full: HLL
+128 x 128 x 64 229 -> 243, 250 x 250 x 16 227 -> 238, but 101 x 101 x 102 287
+-> 245, 500 x 500 x 4 251 -> 239, 128 x 128 x 32 116 -> 102.  Kernel timing
+keeps the launches it accounts for.
 */
-bool flat_step(const pamhd_handle* h)
+bool flat_step(const pamhd_handle* h, int solver)
 {
 	if (h->timing) return false;
-	return h->tune.flat >= 0 ? h->tune.flat == 1 : h->g.n <= 1ll << 20;
+	if (h->tune.flat >= 0) return h->tune.flat == 1;
+	const GridDev& g = h->g;
+	if (h->bg && (solver == RUSANOV || solver == HLL_ATHENA) && g.n > 1ll << 19 && g.nz >= 16) {
+		const long long tiles = (long long)((g.nx + 127) / 128 * 128) * ((g.ny + 1) / 2 * 2) * g.nz;
+		if (16 * tiles <= 17 * g.n) return false;
+	}
+	return g.n <= 1ll << 20;
 }
 
 bool stream_captures(hipStream_t st)
@@ -4886,7 +4900,7 @@ int do_step(pamhd_handle* h, int solver, double max_dt, double cfl, int refits,
 	}
 	StepStatus* prev = h->status + h->last;
 	StepStatus* next = h->status + (1 - h->last);
-	const bool flat = flat_step(h);
+	const bool flat = flat_step(h, solver);
 	if (flat) {
 		const bool report = dt_taken != nullptr;
 		const int e = h->precision == PAMHD_MIXED

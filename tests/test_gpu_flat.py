@@ -11,7 +11,8 @@ import oracle_lib as O
 
 SOLVERS = [("rusanov", O.RUSANOV), ("hll-athena", O.HLL), ("hlld-athena", O.HLLD),
            ("roe-athena", O.ROE)]
-SHAPES = [(1, 1, 1), (5, 3, 4), (63, 2, 2), (64, 4, 1), (257, 1, 1), (17, 15, 1), (1, 1, 300)]
+SHAPES = [(1, 1, 1), (5, 3, 4), (63, 2, 2), (64, 4, 1), (257, 1, 1), (17, 15, 1), (1, 1, 300),
+          (65, 30, 1), (64, 8, 8)]
 
 
 def _state(cells, seed=5):
@@ -54,6 +55,28 @@ def test_flat_fp64_bit_exact_vs_oracle(gpu, cells, name, sid):
         assert g.run(name, 0.3, 0.0, 1e9, max_steps=4) == (steps, t)
         np.testing.assert_array_equal(g.download(), ref)
         assert g.last_flux_calcs() == 3 * n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cells", [(128, 128, 32), (128, 128, 33), (130, 128, 33)])
+@pytest.mark.parametrize("name", ["rusanov", "hll-athena"])
+def test_background_steps_match_the_flat_step(gpu, cells, name):
+    """the default step with a background field around 2^19 cells, where
+    grids of full tiles leave the flat step, against the flat step"""
+    from pamhd_amd import solver as S
+    state, length, gamma, mu0 = _state(cells)
+    bg = 0.1 * np.random.default_rng(3).normal(size=(9, state.shape[1]))
+    out = []
+    for flat in (True, False):
+        with S.Grid(cells, length, gamma, mu0) as g:
+            if flat:
+                g.set_launch(128)
+            g.set_background_faces(bg)
+            g.upload(state)
+            print("cells", cells, name, "flat", flat, flush=True)
+            out.append((g.run(name, 0.3, 0.0, 1e9, max_steps=3), g.max_signal_speeds(), g.download()))
+    assert out[0][:2] == out[1][:2]
+    np.testing.assert_array_equal(out[0][2], out[1][2])
 
 
 @pytest.mark.gpu
