@@ -34,6 +34,7 @@ flux array holds FP32 values.  HLLD accumulates in marches instead
 #include <vector>
 
 #include "pamhd_mi355x.h"
+#include "march.hpp"
 #include "poisson.hpp"
 #include "riemann.hpp"
 #include "plain1d.hpp"
@@ -4156,33 +4157,6 @@ FlatDiv flat_div(unsigned d)
 	while ((1u << lg) < d) lg++;
 	const unsigned sh = 28 + lg;
 	return FlatDiv{(unsigned)(((1ull << sh) / d) + 1), sh};
-}
-
-/*
-Cells per march of a pass over `blocks` blocks of lines with nd cells each,
-at most `most`, when `resident` blocks run on a CU at once: a march of km
-cells costs about km + 1.5 faces, and the blocks run in
-ceil(blocks * chunks / (256 * resident)) rounds, so a fixed km leaves CUs
-idle in the last round or altogether.  FP64 HLLD step, 32-cell marches ->
-this rule: 128^3 545 -> 412 us, 192^3 1493 -> 1387 us, 256^3 within 1 %
-(there VALU issue is the bound whatever the rounds).
-*/
-int march_cells(unsigned blocks, int nd, int resident, int most)
-{
-	const long long slots = 256ll * resident;
-	int best = 1;
-	double best_cost = 1e300;
-	for (int chunks = 1; chunks <= nd; chunks++) {
-		const int km = (nd + chunks - 1) / chunks;
-		if (km > most) continue;
-		const double cost = (double)((blocks * (long long)chunks + slots - 1) / slots) * (km + 1.5);
-		if (cost < best_cost) {
-			best_cost = cost;
-			best = km;
-		}
-		if (km == 1) break;
-	}
-	return best;
 }
 
 /*
