@@ -423,7 +423,9 @@ int pamhd_set_slabs(pamhd_handle* h, int slabs);
 Per-kernel device-time accounting: when enabled, each launch of the handle is
 bracketed by HIP events on its stream.  pamhd_kernel_time synchronises and
 returns the accumulated milliseconds and launch count of one kernel:
-"dt", "flux_pass", "update" or "refit".  Enabling resets the totals.
+"dt", "flux_pass", "update" or "refit" (the flat step computes the step
+length with its faces and needs "dt" only after another kind of step).
+Enabling resets the totals.
 (No counterpart in the reference, which has no timers; used by the
 benchmark for the roofline figure.)
 */

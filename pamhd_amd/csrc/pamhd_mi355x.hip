@@ -4223,12 +4223,10 @@ HLL 90 -> 84, 256 x 256 x 16 196 -> 186, 1024 x 1024 x 1 180 -> 181).  With a
 background field (Rusanov and HLL) both sides fetch it per face, and from
 2^19 cells on the column update gains if its 128 x 2 tiles are full: HLL
 128 x 128 x 64 229 -> 243, 250 x 250 x 16 227 -> 238, but 101 x 101 x 102 287
--> 245, 500 x 500 x 4 251 -> 239, 128 x 128 x 32 116 -> 102.  Kernel timing
-keeps the launches it accounts for.
+-> 245, 500 x 500 x 4 251 -> 239, 128 x 128 x 32 116 -> 102.
 */
 bool flat_step(const pamhd_handle* h, int solver)
 {
-	if (h->timing) return false;
 	if (h->tune.flat >= 0) return h->tune.flat == 1;
 	const GridDev& g = h->g;
 	if (h->bg && (solver == RUSANOV || solver == HLL_ATHENA) && g.n > 1ll << 19 && g.nz >= 16) {
@@ -4253,20 +4251,27 @@ int launch_flat(pamhd_handle* h, int solver, hipStream_t st, double max_dt, doub
 	DtRec* rec = reinterpret_cast<DtRec*>(h->dt);
 	/* a captured step may run after any other one: it reduces the speeds
 	   itself, and so does the step after the capture */
-	if (!h->lag_ok || captured) lag_kernel<<<1, NSLOT, 0, st>>>(prev, next, rec);
+	if (!h->lag_ok || captured) {
+		TimedLaunch t(h, st, K_DT);
+		lag_kernel<<<1, NSLOT, 0, st>>>(prev, next, rec);
+	}
 	h->lag_ok = false;
 	const FlatGrid fg{flat_div((unsigned)h->g.nx), flat_div((unsigned)h->g.ny)};
 	const unsigned nb = (unsigned)((h->g.n + FLAT - 1) / FLAT);
 	const double* s = h->state[h->cur];
 #define FLUX(SV) flat_flux_kernel<SV, T><<<3 * nb, FLAT, 0, st>>>(h->g, fg, s, h->bg, h->flux, rec, cfl, \
 	max_dt, fixed_dt, next)
-	switch (solver) {
-	case RUSANOV: FLUX(RUSANOV); break;
-	case HLL_ATHENA: FLUX(HLL_ATHENA); break;
-	case HLLD_ATHENA: FLUX(HLLD_ATHENA); break;
-	default: FLUX(ROE_ATHENA); break;
+	{
+		TimedLaunch t(h, st, K_FLUX);
+		switch (solver) {
+		case RUSANOV: FLUX(RUSANOV); break;
+		case HLL_ATHENA: FLUX(HLL_ATHENA); break;
+		case HLLD_ATHENA: FLUX(HLLD_ATHENA); break;
+		default: FLUX(ROE_ATHENA); break;
+		}
 	}
 #undef FLUX
+	TimedLaunch t(h, st, K_UPDATE);
 	flat_update_kernel<<<nb + 1, FLAT, 0, st>>>(h->g, fg, s, h->state[1 - h->cur], h->flux, refits,
 		std::is_same_v<T, double> ? h->pe_out : nullptr, next, clear, rec, h->host_dt,
 		report ? h->host_status : nullptr);

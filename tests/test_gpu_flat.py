@@ -146,6 +146,34 @@ def test_flat_reports_the_first_failing_face(gpu):
                 g.check()
 
 
+def _launches(g, steps=5):
+    """dt, flux_pass and update launches of `steps` steps (the step length is
+    a launch of every step but the flat one)"""
+    g.step("hlld-athena", 1e300, 0.3)
+    g.enable_timing(True)
+    for _ in range(steps):
+        g.step("hlld-athena", 1e300, 0.3)
+    n = tuple(g.kernel_time(k)[1] for k in ("dt", "flux_pass", "update"))
+    ms = [g.kernel_time(k)[0] for k in ("flux_pass", "update")]
+    g.enable_timing(False)
+    assert min(ms) > 0
+    return n
+
+
+@pytest.mark.gpu
+def test_kernel_timing_of_the_flat_step(gpu):
+    """timing accounts the launches that untimed steps make"""
+    from pamhd_amd import solver as S
+    cells = (20, 9, 7)
+    state, length, gamma, mu0 = _state(cells)
+    with S.Grid(cells, length, gamma, mu0) as g:
+        g.upload(state)
+        g.timestep("hlld-athena", 0.0, 0.3)
+        assert _launches(g) == (0, 5, 5)
+        g.set_launch(65, 8, 4)
+        assert _launches(g) == (5, 5, 5)
+
+
 @pytest.mark.gpu
 def test_flat_step_replays_in_a_graph(gpu):
     """two captured steps, replayed with eager steps in between"""
