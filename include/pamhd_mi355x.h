@@ -391,7 +391,8 @@ int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen,
    on grids without a background field; bit 1 is then ignored), bit 7 = the
    flat step: one launch for all faces and one for all cells whatever the
    grid's size (the default of grids too small for marches to fill the GPU;
-   the other bits and arguments are then ignored);
+   the other bits and arguments are then ignored; without bit 7 the flat
+   step is off on every grid until pamhd_set_fused_step(h, -1, 0));
    update_remap bits 0 and 1 the same
    orders for the update pass (bit 0 only for the z-marching update) and,
    for the z-marching update, bits 2-4 its tile (0: 64 x 4, 1: 128 x 2,
@@ -407,7 +408,9 @@ int pamhd_set_launch(pamhd_handle* h, int flux_remap, int update_kz, int update_
    place (no flux array); 1 and 2 keep only the two field components of
    each face the constrained-transport edge terms use (6 doubles per cell)
    and finish with a pass that updates the face field and refits the
-   energy.  -1 (the default) picks 2; pamhd_autotune times them all.
+   energy.  -1 (the default) picks 2 and lets grids of up to 2^20 cells take
+   the flat step (of any solver; 0 to 2 turn it off, pamhd_set_launch);
+   pamhd_autotune times them all.
    planes_per_chunk (0 = keep) is the z-extent of mode 1's blocks (1..32)
    or the cells per march of mode 2 (1..32; until it is given they follow
    the grid's size). */
@@ -415,7 +418,8 @@ int pamhd_set_fused_step(pamhd_handle* h, int fused, int planes_per_chunk);
 
 /* Pipelines the flux pass and the per-cell update over `slabs` z-slabs on
    two streams (1 = no pipelining; capped at nz / 2; ignored while kernel
-   timing is on or with the z-marching update).  Identical results.
+   timing is on or with the z-marching update).  More than one slab turns
+   the flat step off, 1 leaves that choice as it was.  Identical results.
    (No counterpart in the reference.) */
 int pamhd_set_slabs(pamhd_handle* h, int slabs);
 

@@ -3826,6 +3826,7 @@ struct pamhd_handle {
 		/* the flat step (two launches): 1 always, 0 never, -1 where the grid
 		   is small (flat_step) and no launch variant was asked for */
 		int flat = -1;
+		bool pipelined = false;   /* slabs > 1 asked for, and not the flat step after it */
 	} tune;
 	/* dt holds the last flux pass's reduced speeds and the other status is
 	   cleared; never true once a step other than a flat one was captured
@@ -4227,6 +4228,7 @@ background field (Rusanov and HLL) both sides fetch it per face, and from
 */
 bool flat_step(const pamhd_handle* h, int solver)
 {
+	if (h->tune.pipelined) return false;
 	if (h->tune.flat >= 0) return h->tune.flat == 1;
 	const GridDev& g = h->g;
 	if (h->bg && (solver == RUSANOV || solver == HLL_ATHENA) && g.n > 1ll << 19 && g.nz >= 16) {
@@ -5873,6 +5875,7 @@ int pamhd_autotune(pamhd_handle* h, int solver, char* buf, size_t buflen, void* 
 		});
 		h->lag_ok = false;
 		h->tune.flat = flat_ms < ms ? 1 : 0;
+		h->tune.pipelined = false;   /* (the comparison included the slabs) */
 		report += "; marches=" + std::to_string(ms) + "ms flat=" + std::to_string(flat_ms) + "ms";
 	}
 	(void)hipEventDestroy(a);
@@ -5908,6 +5911,7 @@ int pamhd_set_launch(pamhd_handle* h, int flux_remap, int update_kz, int update_
 	h->tune.update_remap = update_kz ? (update_remap & 1) : (update_remap & 3);
 	h->tune.update_tile = update_kz ? (update_remap >> 2) % 5 : 0;
 	h->tune.flat = (flux_remap & 128) ? 1 : 0;
+	if (h->tune.flat) h->tune.pipelined = false;
 	return PAMHD_OK;
 }
 
@@ -5934,7 +5938,7 @@ int pamhd_set_slabs(pamhd_handle* h, int slabs)
 	if (!h) return fail(nullptr, PAMHD_E_ARG, "null handle");
 	if (slabs < 1) return fail(h, PAMHD_E_ARG, "slabs must be >= 1");
 	h->tune.slabs = slabs;
-	if (slabs > 1) h->tune.flat = 0;
+	h->tune.pipelined = slabs > 1;
 	return PAMHD_OK;
 }
 

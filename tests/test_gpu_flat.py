@@ -175,6 +175,25 @@ def test_kernel_timing_of_the_flat_step(gpu):
 
 
 @pytest.mark.gpu
+def test_default_step_after_setters_are_undone(gpu):
+    from pamhd_amd import solver as S
+    cells = (20, 9, 7)
+    state, length, gamma, mu0 = _state(cells)
+    flat, other = (0, 5, 5), (5, 5, 5)
+    with S.Grid(cells, length, gamma, mu0) as g:
+        g.upload(state)
+        g.timestep("hlld-athena", 0.0, 0.3)
+        for call, want in ((lambda: g.set_slabs(3), other), (lambda: g.set_slabs(1), flat),
+                           (lambda: g.set_slabs(3), other), (lambda: g.set_fused_step("auto"), other),
+                           (lambda: g.set_launch(128), flat), (lambda: g.set_slabs(3), other),
+                           (lambda: g.set_slabs(1), flat), (lambda: g.set_launch(0, 0, 0), other),
+                           (lambda: g.set_slabs(1), other), (lambda: g.set_fused_step("auto"), flat),
+                           (lambda: g.set_fused_step("passes"), other), (lambda: g.set_fused_step("auto"), flat)):
+            call()
+            assert _launches(g) == want
+
+
+@pytest.mark.gpu
 def test_flat_step_replays_in_a_graph(gpu):
     """two captured steps, replayed with eager steps in between"""
     import torch
