@@ -327,11 +327,9 @@ def ensemble_run(nbox, steps, solver="hll-athena", cfl=0.3, seed=2024, imf_steps
     # the same steps in one persistent launch (last: a cooperative launch is
     # not to precede the other timings) (stages separated by grid-wide
     # barriers), from the same start and tile shape
-    tiles = {"64x4": 0, "32x8": 1, "16x16": 2}
+    tiles = {"64x4": 0, "32x8": 1, "16x16": 2, "256x1": 3}
     with Ensemble(boxes) as e2:
-        shape = tune.split("; chosen ")[-1].strip()
-        if shape in tiles:      # else the default, which autotuning chose
-            e2.set_tile(tiles[shape])
+        e2.set_tile(tiles[tune.split("; chosen ")[-1].strip()])
         e2.timestep(solver, 0.0, cfl, stream=stream)
         e2.run(solver, cfl, 2, use_graph=False, stream=stream)
         torch.cuda.synchronize()

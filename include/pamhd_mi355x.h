@@ -563,7 +563,8 @@ program.)
                first physics error
   autotune     picks the fastest tile shape of the cell kernels (64x4, 32x8,
                16x16 or the default 256x1, consecutive cells) on a copy of
-               the state; set_tile sets one of the first three
+               the state; set_tile sets one (0 to 3 in this order; 3 for
+               boxes of fewer than 2^28 cells, others start with 0)
 */
 int pamhd_ensemble_create(int nbox, const pamhd_grid_desc* grids, const pamhd_physics* physics,
 	const pamhd_solar_wind_desc* solar_winds, pamhd_ensemble** out);

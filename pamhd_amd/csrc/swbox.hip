@@ -1190,9 +1190,17 @@ static int use_tile(BoxSet* s, int tile)
 	return build_blocks(s) == hipSuccess ? PAMHD_OK : PAMHD_E_DEVICE;
 }
 
+/* whether every box's flat index fits T_FLAT's 28 bits */
+static bool flat_tiles_fit(const BoxSet* s)
+{
+	for (const BoxDev& B : s->host)
+		if (B.n >= 1 << 28) return false;
+	return true;
+}
+
 int boxset_set_tile(BoxSet* s, int tile)
 {
-	if (tile < 0 || tile > 2) return PAMHD_E_ARG;
+	if (tile < 0 || tile > T_FLAT || (tile == T_FLAT && !flat_tiles_fit(s))) return PAMHD_E_ARG;
 	return use_tile(s, tile);
 }
 
@@ -1386,8 +1394,7 @@ int boxset_create(BoxSet** out, int nbox, const pamhd_grid_desc* grids, const pa
 		}
 		off += n;
 	}
-	for (const BoxDev& B : s->host)
-		if (B.n >= 1 << 28) s->tile = 0;
+	if (!flat_tiles_fit(s)) s->tile = 0;
 	if ((e = build_blocks(s)) != hipSuccess) return bail(e, "blocks");
 	s->nbnd = (long long)bnd.size();
 	s->ninflow = (long long)inflow.size();
@@ -1646,9 +1653,7 @@ int boxset_autotune(BoxSet* s, int solver, double cfl, int steps, hipStream_t st
 	float best_ms = 1e30f;
 	int rc = PAMHD_OK;
 	report += "tiles:";
-	int shapes = 4;
-	for (const BoxDev& B : s->host)
-		if (B.n >= 1 << 28) shapes = 3;
+	const int shapes = flat_tiles_fit(s) ? T_FLAT + 1 : T_FLAT;
 	for (int t = 0; t < shapes && rc == PAMHD_OK; t++) {
 		if (use_tile(s, t) != PAMHD_OK) {
 			rc = PAMHD_E_DEVICE;

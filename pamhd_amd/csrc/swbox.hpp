@@ -30,8 +30,8 @@ long long boxset_cells(const BoxSet* s, int box);
    flux_calcs, source/mhd/solve.hpp:253-313 */
 long long boxset_faces(const BoxSet* s, int box);
 
-/* tile shape of the cell kernels: 0 = 64x4, 1 = 32x8, 2 = 16x16 (until it
-   is set: 256 consecutive cells) */
+/* tile shape of the cell kernels: 0 = 64x4, 1 = 32x8, 2 = 16x16, 3 = 256x1
+   (256 consecutive cells, the default; boxes of fewer than 2^28 cells) */
 int boxset_set_tile(BoxSet* s, int tile);
 int boxset_tile(const BoxSet* s);
 

@@ -242,6 +242,8 @@ class Ensemble:
         return out
 
     def set_tile(self, tile):
+        """tile shape of the cell kernels: 0 64x4, 1 32x8, 2 16x16, 3 256x1
+        (consecutive cells, the default); identical results"""
         self._check(self._L.pamhd_ensemble_set_tile(self._e, tile))
 
     def autotune(self, solver, time_step_factor, stream=None):

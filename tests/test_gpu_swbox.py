@@ -228,3 +228,25 @@ def test_config_box_runs_and_keeps_inflow(gpu):
     assert np.all(s[0][ct >= 0] > 0)
     sw = ru == O.RULE_SW
     np.testing.assert_array_equal(s[0][sw], sb.number_density * sb.proton_mass)
+
+
+def test_default_tile_can_be_set_again(gpu):
+    from pamhd_amd import _lib
+    from pamhd_amd.swbox import Ensemble
+    boxes = _ensemble_boxes()
+    outs = []
+    for tiles in ((), (1, 3)):
+        with Ensemble(boxes) as e:
+            e.timestep("hll-athena", 0.0, 0.3)
+            for t in tiles:
+                e.set_tile(t)
+                e.run("hll-athena", 0.3, 2)
+            if not tiles:
+                e.run("hll-athena", 0.3, 4)
+            for t in (-1, 4):
+                with pytest.raises(_lib.PamhdError):
+                    e.set_tile(t)
+            e.check()
+            outs.append([e.download(q) for q in range(len(boxes))])
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)
