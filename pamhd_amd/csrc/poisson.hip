@@ -13,7 +13,7 @@ own in whole cache lines.  Kernels:
   restrict_residual_kernel  both of these at once, for pairs coarsened by 2
                    in every dimension (no r array)
   prolong_kernel   fine phi += trilinear interpolation of coarse phi
-  prolong8_kernel  the same, a thread per coarse cell and its 8 children
+  prolong8_kernel  the same, a thread per coarse cell, its black children only
   prolong_packed_kernel  the same between packed levels, two coarse cells a
                    thread, the black children only
   coarse_kernel    all sweeps of a small level inside one block, in LDS
@@ -359,13 +359,14 @@ __global__ __launch_bounds__(PBX * PBY) void restrict_residual_kernel(Tiles T, L
 }
 
 /* prolongation for level pairs coarsened by 2 in every dimension: a thread
-   adds the interpolation to the 8 children of its coarse cell from the 27
-   coarse values around it, each child's terms in the order of
-   prolong_kernel.  Before red-black sweeps only the black children are
-   needed (BLACK): the first red pass replaces every red value from black
-   ones.  That halves the traffic on the fine level: 54 us instead of 72 to
-   256^3 cells. */
-template <bool BLACK>
+   adds the interpolation to the black children of its coarse cell from the
+   27 coarse values around it, each child's terms in the order of
+   prolong_kernel.  The red children are not needed: such a fine level is
+   even in every dimension, so both smoothers sweep it red-black and the
+   first red pass replaces every red value from black ones (a level whose
+   spacings' squares overflow is not swept, but then neither is the coarse
+   one, whose phi stays 0).  That halves the traffic on the fine level:
+   54 us instead of 72 to 256^3 cells. */
 __global__ __launch_bounds__(PBX * PBY) void prolong8_kernel(Tiles T, LevelArgs F, LevelArgs C,
 	double* __restrict__ phi, const double* __restrict__ cphi)
 {
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(PBX * PBY) void prolong8_kernel(Tiles T, LevelArgs 
 	for (int c = 0; c < 2; c++)
 	for (int b = 0; b < 2; b++)
 	for (int a = 0; a < 2; a++) {
-		if (BLACK && ((a + b + c) & 1) == 0) continue;
+		if (((a + b + c) & 1) == 0) continue;
 		/* the parent (index 1) and its neighbour on the child's side */
 		const int pa[2] = {1, a ? 2 : 0}, pb[2] = {1, b ? 2 : 0}, pc[2] = {1, c ? 2 : 0};
 		double s = 0;
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(PBX * PBY) void prolong8_kernel(Tiles T, LevelArgs 
 }
 
 /*
-prolong8_kernel<true> from a packed level: a thread takes the coarse cells
+prolong8_kernel from a packed level: a thread takes the coarse cells
 2t and 2t + 1, whose values and neighbours are consecutive over the threads
 in each colour's half, where a thread a cell makes every one of its 27 loads
 two half-used pieces, and writes two black children at a time.  To 256^3
@@ -1329,14 +1330,12 @@ void mg_vcycle(PoissonMG& mg, hipStream_t st, int l)
 			F.r, C.f, C.phi);
 	}
 	mg_vcycle(mg, st, l + 1);
-	if (by2 && F.packed && C.packed) {
+	if (by2 && C.packed) {
 		const Tiles TP = level_tiles(C, 2);
 		prolong_packed_kernel<<<blocks_of(TP), dim3(PBX, PBY, 1), 0, st>>>(TP, args_of(F), args_of(C),
 			F.phi, C.phi);
-	} else if (by2 && rb_ok(F) && F.diag != 0) {
-		prolong8_kernel<true><<<blocks_of(TC), dim3(PBX, PBY, 1), 0, st>>>(TC, args_of(F), args_of(C), F.phi, C.phi);
 	} else if (by2) {
-		prolong8_kernel<false><<<blocks_of(TC), dim3(PBX, PBY, 1), 0, st>>>(TC, args_of(F), args_of(C), F.phi, C.phi);
+		prolong8_kernel<<<blocks_of(TC), dim3(PBX, PBY, 1), 0, st>>>(TC, args_of(F), args_of(C), F.phi, C.phi);
 	} else {
 		prolong_kernel<<<blocks_of(TF), dim3(PBX, PBY, 1), 0, st>>>(TF, args_of(F), args_of(C), q,
 			F.phi, C.phi);
