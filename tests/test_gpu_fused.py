@@ -73,7 +73,7 @@ def test_fused_chunks_match_two_pass(gpu, mode, kc):
     np.testing.assert_array_equal(sa, sb)
 
 
-@pytest.mark.parametrize("cells", [(64, 12, 10), (70, 13, 33)])
+@pytest.mark.parametrize("cells", [(64, 12, 10), (70, 13, 33), (5, 3, 4), (16, 12, 10), (40, 40, 1), (1, 1, 8)])
 def test_fused_mixed_matches_two_pass_mixed(gpu, cells):
     print("cells", cells, flush=True)
     b, nb, tb, _, _ = _run(cells, 6, "passes", precision="mixed")

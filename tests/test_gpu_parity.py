@@ -113,6 +113,31 @@ def test_grid_steps_face_varying_background(gpu, name, sid):
     np.testing.assert_array_equal(out, ref)
 
 
+@pytest.mark.parametrize("cells", [(70, 9, 13), (130, 11, 21)])
+@pytest.mark.parametrize("name,sid,background", [(*s, False) for s in SOLVERS] + [(*s, True) for s in SOLVERS[:2]])
+def test_large_grid_launches_bit_exact(gpu, name, sid, cells, background):
+    """the launches that grids too large for the flat step take by default
+    (fewer than 16 planes: per-cell update), on shapes with partial tiles,
+    with and without a background field that differs on every face (Rusanov
+    and HLL use it)"""
+    from pamhd_amd import solver as S
+    state, length, gamma, mu0 = _vortex(cells, seed=22)
+    n = state.shape[1]
+    bg = np.random.default_rng(6).uniform(-0.2, 0.2, size=(9, n)) if background else None
+    ref = state.copy()
+    st, steps_o, t_o = O.run_periodic(O.make_grid(cells, length, gamma, mu0, bg), sid, 0.3, 0.0, 1e9, ref,
+                                      max_steps=4)
+    assert st == 0
+    with S.Grid(cells, length, gamma, mu0) as g:
+        g.set_launch(65, 8, 4)
+        g.upload(state)
+        if background:
+            g.set_background_faces(bg)
+        print("cells", cells, name, "background", background, flush=True)
+        assert g.run(name, 0.3, 0.0, 1e9, max_steps=4) == (steps_o, t_o)
+        np.testing.assert_array_equal(g.download(), ref)
+
+
 @pytest.mark.parametrize("variant", [(0, 0, 0), (1, 0, 1), (0, 4, 0), (1, 8, 1), (0, 32, 1),
                                      (2, 0, 2), (3, 0, 3), (4, 0, 0), (7, 0, 2),
                                      (0, 8, 4), (1, 4, 9), (0, 16, 8), (0, 8, 12), (1, 16, 17)])
