@@ -4222,16 +4222,17 @@ cells they leave SIMDs without a wave.  us per step, marches -> flat:
 so all cross over at about 100^3 cells, in mixed precision too (512 x 512 x 2
 HLL 90 -> 84, 256 x 256 x 16 196 -> 186, 1024 x 1024 x 1 180 -> 181).  With a
 background field (Rusanov and HLL) both sides fetch it per face, and from
-2^19 cells on the column update gains if its 128 x 2 tiles are full: HLL
-128 x 128 x 64 229 -> 243, 250 x 250 x 16 227 -> 238, but 101 x 101 x 102 287
--> 245, 500 x 500 x 4 251 -> 239, 128 x 128 x 32 116 -> 102.
+about 9 10^5 cells on the column update gains if its 128 x 2 tiles are full:
+HLL 128 x 128 x 48 177 -> 173, x 56 207 -> 204, x 60 221 -> 223, x 64 234 ->
+245, 256 x 250 x 16 231 -> 239, but 101 x 101 x 102 287 -> 245, 500 x 500 x 4
+251 -> 239.
 */
 bool flat_step(const pamhd_handle* h, int solver)
 {
 	if (h->tune.pipelined) return false;
 	if (h->tune.flat >= 0) return h->tune.flat == 1;
 	const GridDev& g = h->g;
-	if (h->bg && (solver == RUSANOV || solver == HLL_ATHENA) && g.n > 1ll << 19 && g.nz >= 16) {
+	if (h->bg && (solver == RUSANOV || solver == HLL_ATHENA) && g.n > 7ll << 17 && g.nz >= 16) {
 		const long long tiles = (long long)((g.nx + 127) / 128 * 128) * ((g.ny + 1) / 2 * 2) * g.nz;
 		if (16 * tiles <= 17 * g.n) return false;
 	}
