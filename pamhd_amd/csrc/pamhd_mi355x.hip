@@ -7,7 +7,7 @@ Data layout in HBM (structure of arrays, FP64, component-major):
             rho, m_x, m_y, m_z, E, B_x(i-1/2), B_y(j-1/2), B_z(k-1/2)
   flux      24 * n values: dt * F_q of the d-face owned by each cell
             (d-major, then component, then cell), written by the flux pass
-            and read by the update pass (FP64, or FP32 in mixed precision)
+            and read by the update pass (doubles, in mixed precision too)
   bg        optional 9 * n doubles of background field on the positive faces
   status[2] per-pass reductions (max signal speed per dimension, count of
             faces with speed <= 0, first physics error) feeding the lagged
@@ -17,9 +17,8 @@ One step = dt_kernel (1 thread: lagged CFL step from the previous pass) ->
 flux_pass_kernel (one thread per face, all faces of one dimension in a
 z-slab of blocks) -> update_cell_kernel or update_column_kernel (one thread
 per cell, or column tiles marching in z: constrained-transport face update,
-conserved update, constant-pressure energy refits).  In mixed precision the
-flux array holds FP32 values.  HLLD accumulates in marches instead
-(launch_accumulate), and grids of up to 2^20 cells step in two launches
+conserved update, constant-pressure energy refits).  HLLD accumulates in
+marches instead (launch_accumulate), and most grids of up to 2^20 cells step in two launches
 (flat_step).
 */
 #include <hip/hip_runtime.h>
