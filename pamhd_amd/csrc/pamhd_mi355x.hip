@@ -18,8 +18,8 @@ flux_pass_kernel (one thread per face, all faces of one dimension in a
 z-slab of blocks) -> update_cell_kernel or update_column_kernel (one thread
 per cell, or column tiles marching in z: constrained-transport face update,
 conserved update, constant-pressure energy refits).  HLLD accumulates in
-marches instead (launch_accumulate), and most grids of up to 2^20 cells step in two launches
-(flat_step).
+marches instead (launch_accumulate), and most grids of up to 2^20 cells step
+in two launches (flat_step).
 */
 #include <hip/hip_runtime.h>
 
@@ -1367,10 +1367,14 @@ __global__ __launch_bounds__(NSLOT) void lag_kernel(StepStatus* cur, StepStatus*
 }
 
 /* cells / FLAT blocks update the cells, the last block ends the pass; host
-   (pinned, may be null) receives the step length and the error.  The
-   blocks take the cells in the XCD-aware order, so that the rows and planes
-   around a block's are read through the same L2: HLL mixed, 512 x 512 x 2
-   103 -> 89 us a step, 512 x 512 x 4 200 -> 186 */
+   (pinned, may be null) receives the step length and the error.  Above two
+   blocks a CU the blocks take the cells in the XCD-aware order, so that the
+   rows and planes around a block's are read through the same L2: HLL mixed,
+   512 x 512 x 2 103 -> 84 us a step, 512 x 512 x 4 200 -> 184, 40 x 64 x 80
+   48 -> 44; with fewer blocks it gains nothing (48^3 29.9 -> 29.5, 128 x 128
+   x 8 30.8 -> 31.4, 128 x 128 x 4 22.9 -> 23.8) */
+constexpr unsigned FLAT_XCD = 2 * 256;   /* blocks up to which the order is the plain one */
+
 __global__ __launch_bounds__(FLAT) void flat_update_kernel(GridDev g, FlatGrid fg,
 	const double* __restrict__ s, double* __restrict__ out, const double* __restrict__ P, int refits,
 	double* __restrict__ pe, StepStatus* cur, StepStatus* other, DtRec* rec, double* host_dt,
@@ -1393,7 +1397,8 @@ __global__ __launch_bounds__(FLAT) void flat_update_kernel(GridDev g, FlatGrid f
 		}
 		return;
 	}
-	const int c = (int)logical_block(blockIdx.x, gridDim.x - 1) * FLAT + threadIdx.x;
+	const unsigned nb = gridDim.x - 1;
+	const int c = (int)(nb > FLAT_XCD ? logical_block(blockIdx.x, nb) : blockIdx.x) * FLAT + threadIdx.x;
 	if (c >= (int)g.n) return;
 	int i, j, k;
 	fg.cell(g, c, i, j, k);
@@ -1879,8 +1884,8 @@ path, each finishing its direction's part of update_mhd_state's conserved
 update (source/mhd/solve.hpp:1503-1614) instead of storing face fluxes:
 
   acc_x_kernel      x-faces, a wave per 64 cells of a plane walking km planes
-                    along z, or y on flat grids (the left part of lane l is lane l - 1's, the
-                    face of lane l + 1 comes one lane down; the rows'
+                    along z, or y on flat grids (the left part of lane l is
+                    lane l - 1's, the face of lane l + 1 comes one lane down; the rows'
                     left-edge parts and right-edge face fluxes are computed
                     for all km planes before the march); writes
                     out = U + x terms (8 values: rho, m, E, cell-centred B)

@@ -12,7 +12,7 @@ import oracle_lib as O
 SOLVERS = [("rusanov", O.RUSANOV), ("hll-athena", O.HLL), ("hlld-athena", O.HLLD),
            ("roe-athena", O.ROE)]
 SHAPES = [(1, 1, 1), (5, 3, 4), (63, 2, 2), (64, 4, 1), (257, 1, 1), (17, 15, 1), (1, 1, 300),
-          (65, 30, 1), (64, 8, 8)]
+          (65, 30, 1), (64, 32, 64), (67, 31, 64)]
 
 
 def _state(cells, seed=5):
