@@ -5055,9 +5055,10 @@ int pamhd_create_bounded(const pamhd_grid_desc* grid, const pamhd_physics* physi
 	d.smax = 0;
 	d.opt = nullptr;
 	h->cell_type.assign(cell_type, cell_type + n);
-	for (long long q = 0; q < 3 * n; q++)
-		if (var_type[q] == 4 && cell_type[q % n] >= 1) h->normal_copied = true;
-	h->normal_written = h->normal_copied;
+	int copied = 0;
+	for (int v = 0; v < 3; v++)
+		for (long long c = 0; c < n; c++) copied |= (var_type[v * n + c] == 4) & (cell_type[c] >= 1);
+	h->normal_copied = h->normal_written = copied != 0;
 	*out = h;
 	return PAMHD_OK;
 }
